@@ -122,12 +122,12 @@ int m5k_gemm_i8(const int8_t* a, const int8_t* b, int64_t m, int64_t n, int64_t 
                 void* stream);
 
 /*
- * The same W8A8 linear as m5k_gemm_i8 for short M: each output tile (256 x 256, or 256 x 64
- * (k <= 8192) or 256 x 128 when the tiles x splits fit in one round) is split over `splits`
- * contiguous ranges of K (1..64), the raw INT32 partial tiles go to workspace[splits][m][n]
- * (int32, caller-owned, at least splits*m*n elements), and a second kernel sums them in
- * split order and applies the identical epilogue.  INT32 sums are exact, so c is bit-identical
- * to m5k_gemm_i8's.  Needs k % 16 == 0 and 16-byte aligned a/b (any operand size).  Same
+ * The same W8A8 linear as m5k_gemm_i8 for short M: each output tile may be split over up to
+ * `splits` contiguous ranges of K (1..64).  The library takes the tile and the number of ranges
+ * that it expects to be fastest; with one range it is m5k_gemm_i8's launch and the workspace stays
+ * untouched.  Otherwise the raw INT32 partial tiles go to workspace[splits][m][n] (int32,
+ * caller-owned, at least splits*m*n elements), and a second kernel sums them in split order and
+ * applies the identical epilogue.  INT32 sums are exact, so c is bit-identical to m5k_gemm_i8's.  Needs k % 16 == 0 and 16-byte aligned a/b (any operand size).  Same
  * contract as metal.gemm(a, b, "int8", ...) (src/m5kernels/metal.py:158-269); the split is
  * this library's schedule for few-tile shapes (one or two 256-row tile rows).
  */
@@ -167,7 +167,7 @@ int m5k_gemm_i8_splitk_noalloc(const int8_t* a, const int8_t* b, int64_t m, int6
  *   3  quad: 256 x 256 tiles on four waves of 128 x 128 (I8 only; only when forced, below);
  * and *full_tiles is -1 unless the schedule is 1.  Every m5k_gemm_* entry point makes this
  * choice with the device's CU count for operands on the direct-to-LDS path (row bytes a
- * multiple of 16, 16-byte aligned bases); the others run the plain schedule.  Results are
+ * multiple of 16, 16-byte aligned bases) whose tile is 0 in m5k_gemm_tile_plan.  Results are
  * bit-identical under every schedule.  M5K_GEMM_MIXED_TILES=0 / M5K_GEMM_NARROW_TILES=0 in
  * the environment switch schedule 1 / 2 off.
  */
@@ -182,9 +182,25 @@ int m5k_gemm_launch_plan(int ab_dtype, int64_t m, int64_t n, int cus, int* sched
  * (src/m5kernels/cli.py:66-151); this is the gfx950 knob the harness tuner searches instead.
  * The setting is thread-local, so other host threads keep their own plan; for tools outside the
  * process, M5K_GEMM_SCHEDULE=plain|mixed|narrow|quad in the environment does the same when no thread
- * setting is made.  Results are bit-identical under every schedule.
+ * setting is made.  Results are bit-identical under every schedule.  Under a forced schedule aligned
+ * operands run that schedule's 256-row tiles whatever m5k_gemm_tile_plan would choose.
  */
 int m5k_gemm_set_schedule(int schedule, int* previous);
+
+/*
+ * Tile of the MFMA GEMMs for an [m,n,k] product (host only, launches nothing; no counterpart in the
+ * reference).  `aligned`: row bytes a multiple of 16 and at most 2^23, 16-byte aligned bases.  *tile
+ * receives
+ *   0  the 256-row schedules of m5k_gemm_launch_plan;
+ *   1  128 x 128 tiles, K over two groups of waves;
+ *   2  64 x 64 tiles, two workgroups per CU, K over two groups of waves;
+ *   3  64 x 64 tiles with longer stages, the same sums;
+ *   4  16 columns per workgroup, K over eight waves (m <= 32).
+ * INT8 results are bit-identical under every tile.  Float results (FP32 sums) are the same bits for
+ * tiles 1 to 3, and for tile 0 under every schedule; between these groups and tile 4 the order of the
+ * sum differs.  Float rows of under 1 KiB always take tile 0.
+ */
+int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int* tile);
 
 /*
  * Raw INT32 accumulators of the W8A8 GEMM (test hook for bit-exact parity):
@@ -306,6 +322,14 @@ int m5k_projection_qk_rope(const void* a, const void* b, int ab_dtype, int64_t m
  */
 int m5k_qk_norm_rope(const void* projected, int64_t m, int64_t n, const void* gamma, const void* cos,
                      const void* sin, int rope_half, float epsilon, void* y, void* stream);
+
+/*
+ * The same for a BF16 projection in the grouped layout of m5k_projection_qkv_rope, [m, heads*3*128]:
+ * Q and K blocks are normalized and rotated, V blocks copied, to [heads, m, 128] each (16-byte aligned).
+ */
+int m5k_qkv_norm_rope(const void* projected, int64_t m, int64_t heads, const void* q_gamma, const void* k_gamma,
+                      const void* cos, const void* sin, int rope_half, float epsilon, void* q_out, void* k_out,
+                      void* v_out, void* stream);
 
 /*
  * Grouped Q/K/V projection in the H3 runtime's native layout

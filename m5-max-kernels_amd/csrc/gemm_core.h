@@ -59,13 +59,15 @@ constexpr int GROUP_M = 4;             // tile-rows per raster band
 // TN is the tile's column count: BN for the full tile, less for the narrower tiles that refill
 // a partial last round or make the tile count a whole number of rounds.  B rows are moved in
 // whole 16-row groups per wave; rows past TN load nothing (their LDS rows are never read).
-template <int WAVES_M_, int WAVES_N_, int TN_ = BN>
+// TM is its row count: BM here, less for the ring kernels (gemm_ring.h), which use a Grid for the
+// geometry of their epilogue.
+template <int WAVES_M_, int WAVES_N_, int TN_ = BN, int TM_ = BM>
 struct Grid {
   static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
   static constexpr int WAVES = WAVES_M * WAVES_N;
   static constexpr int THREADS = 64 * WAVES;
-  static constexpr int TN = TN_;
-  static constexpr int WM = BM / WAVES_M, WN = TN / WAVES_N;
+  static constexpr int TN = TN_, TM = TM_;
+  static constexpr int WM = TM / WAVES_M, WN = TN / WAVES_N;
   static constexpr int DMA_ROWS = BM / WAVES;       // A rows one wave DMAs per stage
   static constexpr int DMA_INSTR = DMA_ROWS / 8;    // 1 KiB (8 rows of 128 B) per instruction
   static constexpr int DMA_ROWS_B = (TN / WAVES + 15) / 16 * 16;  // B rows one wave DMAs per stage
@@ -75,7 +77,6 @@ using Grid4 = Grid<2, 2>;
 using Grid8 = Grid<2, 4>;
 using Grid8Half = Grid<4, 2, BN / 2>;     // 256 x 128 tile, 8 waves of 64 x 64
 using Grid8Narrow = Grid<4, 2, 7 * BN / 8>;  // 256 x 224 tile, 8 waves of 64 x 112 (16 x 16 modes)
-using Grid8Skinny = Grid<8, 1, BN / 4>;      // 256 x 64 tile, 8 waves of 32 x 64 (split-K of short M)
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 template <int MODE>
@@ -181,8 +182,14 @@ constexpr int TILE16_STRIDE = BN + 8;
 // 132 KiB, then the tile's row and column scales, 2 KiB).  The DMA writes are inline asm with
 // "memory" clobbers and every consumer sits behind an explicit wait and barrier, so one array
 // serves all stages.
-constexpr int EPI_SCALES_OFFSET = BM * TILE16_STRIDE * 2;
-constexpr int EPI_BYTES = EPI_SCALES_OFFSET + (BM + BN) * 4;
+// The ring kernels' smaller tiles (TM < BM) keep the same layout with rows of TN + 8 elements.
+template <class G>
+struct EpiLayout {
+  static constexpr int STRIDE = (G::TM == BM ? BN : G::TN) + 8;
+  static constexpr int SCALES_OFFSET = G::TM * STRIDE * 2;
+  static constexpr int BYTES = SCALES_OFFSET + (G::TM + (G::TM == BM ? BN : G::TN)) * 4;
+};
+constexpr int EPI_BYTES = EpiLayout<Grid<2, 4>>::BYTES;
 constexpr int LDS_BYTES = NST * 2 * STAGE_BYTES > EPI_BYTES ? NST * 2 * STAGE_BYTES : EPI_BYTES;
 __shared__ __attribute__((aligned(16))) uint8_t g_lds[LDS_BYTES];
 
@@ -663,8 +670,10 @@ __device__ __forceinline__ void mainloop_dma(const uint8_t* __restrict__ A, cons
   stage_barrier();
 }
 
-// Register-staged main loop for rows that are not 16-byte multiples (small, odd K): bytes
-// are loaded one at a time with exact bounds, then stored to the same swizzled layout.
+// Register-staged main loop for operands that the direct-to-LDS loads do not take, in the forms
+// that the ring kernels (gemm_ring.h) do not serve: FP32, FP8 at a misaligned base, and the raw INT32
+// accumulators.  Bytes are loaded one at a time with exact bounds, then stored to the same swizzled
+// layout.
 template <int MODE, class G>
 __device__ __forceinline__ void mainloop_staged(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M,
                                                 int N, int64_t Kb, int tile_m0, int tile_n0, AccTile<MODE, G>& acc) {
@@ -745,15 +754,15 @@ struct AccGeom {
 // counts stay exact.
 template <class G>
 struct TileScalePrefetch {
-  static constexpr int PER = (BM + G::TN + G::THREADS - 1) / G::THREADS;  // scales per thread
+  static constexpr int PER = (G::TM + G::TN + G::THREADS - 1) / G::THREADS;  // scales per thread
   float v[PER];
   __device__ __forceinline__ TileScalePrefetch(const float* __restrict__ sa, const float* __restrict__ sb, int M,
                                                int N, int m0, int n0) {
     if constexpr (PER == 1) {
       // One scale per thread: a single load from either vector (the eight-wave grids).
       const int t = threadIdx.x;
-      const int m = m0 + t, n = n0 + t - BM;
-      v[0] = t < BM ? (m < M ? sa[m] : 0.0f) : (t < BM + G::TN && n < N ? sb[n] : 0.0f);
+      const int m = m0 + t, n = n0 + t - G::TM;
+      v[0] = t < G::TM ? (m < M ? sa[m] : 0.0f) : (t < G::TM + G::TN && n < N ? sb[n] : 0.0f);
     } else {
       // Thread t takes row scale t and column scale t (PER == 2: BM == TN == THREADS).
       static_assert(PER == 2 && G::THREADS == BM && G::TN == BM, "two scales per thread: one row, one column");
@@ -770,29 +779,29 @@ struct TileScalePrefetch {
 // scales from the LDS one block row at a time, so the epilogue holds few extra registers.
 template <class G>
 struct TileScales {
-  const float* s;  // rows [0, BM), then columns [BM, BM + G::TN)
+  const float* s;  // rows [0, BM), then columns [BM, G::TM + G::TN)
   __device__ __forceinline__ TileScales(const float* __restrict__ sa, const float* __restrict__ sb, int M, int N,
-                                        int m0, int n0, int tid) {
-    float* w = reinterpret_cast<float*>(g_lds + EPI_SCALES_OFFSET);
-    for (int t = tid; t < BM + G::TN; t += G::THREADS) {
-      const int m = m0 + t, n = n0 + t - BM;
-      w[t] = t < BM ? (m < M ? sa[m] : 0.0f) : (n < N ? sb[n] : 0.0f);
+                                        int m0, int n0, int tid, uint8_t* lds = g_lds) {
+    float* w = reinterpret_cast<float*>(lds + EpiLayout<G>::SCALES_OFFSET);
+    for (int t = tid; t < G::TM + G::TN; t += G::THREADS) {
+      const int m = m0 + t, n = n0 + t - G::TM;
+      w[t] = t < G::TM ? (m < M ? sa[m] : 0.0f) : (n < N ? sb[n] : 0.0f);
     }
     __syncthreads();
     s = w;
   }
-  __device__ __forceinline__ TileScales(const TileScalePrefetch<G>& pre, int tid) {
-    float* w = reinterpret_cast<float*>(g_lds + EPI_SCALES_OFFSET);
+  __device__ __forceinline__ TileScales(const TileScalePrefetch<G>& pre, int tid, uint8_t* lds = g_lds) {
+    float* w = reinterpret_cast<float*>(lds + EpiLayout<G>::SCALES_OFFSET);
 #pragma unroll
     for (int i = 0; i < TileScalePrefetch<G>::PER; ++i) {
       const int t = tid + i * G::THREADS;
-      if (t < BM + G::TN) w[t] = pre.v[i];
+      if (t < G::TM + G::TN) w[t] = pre.v[i];
     }
     __syncthreads();
     s = w;
   }
   __device__ __forceinline__ float row(int r) const { return s[r]; }
-  __device__ __forceinline__ float col(int c) const { return s[BM + c]; }
+  __device__ __forceinline__ float col(int c) const { return s[G::TM + c]; }
 };
 
 // Visit every accumulator element with its global (row, col).

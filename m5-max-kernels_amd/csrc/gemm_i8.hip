@@ -60,6 +60,22 @@ extern "C" int m5k_gemm_launch_plan(int ab_dtype, int64_t m, int64_t n, int cus,
   return M5K_OK;
 }
 
+extern "C" int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int* tile) {
+  clear_error();
+  const char* name = "m5k_gemm_tile_plan";
+  M5K_REQUIRE(tile != nullptr, "%s: null output", name);
+  if (int rc = check_shape(m, n, k, name)) return rc;
+  M5K_REQUIRE(cus > 0, "%s: cus must be positive", name);
+  switch (ab_dtype) {
+    case M5K_I8: *tile = plan_tile(I8, m, n, k, cus, aligned != 0).tile; return M5K_OK;
+    case M5K_U8: *tile = plan_tile(F8, m, n, k, cus, aligned != 0).tile; return M5K_OK;
+    case M5K_BF16: *tile = plan_tile(BF16, m, n, 2 * k, cus, aligned != 0).tile; return M5K_OK;
+    case M5K_F16: *tile = plan_tile(F16, m, n, 2 * k, cus, aligned != 0).tile; return M5K_OK;
+    case M5K_F32: *tile = plan_tile(F32, m, n, 4 * k, cus, aligned != 0).tile; return M5K_OK;
+    default: set_error("%s: ab_dtype must be I8, U8 (FP8 codes), BF16, F16 or F32", name); return M5K_EINVAL;
+  }
+}
+
 extern "C" int m5k_gemm_set_schedule(int schedule, int* previous) {
   clear_error();
   M5K_REQUIRE(schedule >= -1 && schedule <= SCHED_QUAD, "m5k_gemm_set_schedule: schedule %d outside [-1, 3]",

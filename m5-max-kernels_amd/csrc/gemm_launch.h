@@ -1,214 +1,18 @@
-// W8A8 / FP8 / BF16 / FP16 linear layers on gfx950 MFMA with fused epilogues.
-//
-// Contract: src/m5kernels/metal.py:158-269 (gemm) with the epilogue strings of
-// metal.py:88-128:
-//   quantized  C = O(float(acc) * AS[row] * BS[col])            (left to right, FP32)
-//   + bias     C = O(float(acc) * AS[row] * BS[col] + Bias[..])  (before the output cast)
-//   gated      branch = bf16(value); C = bf16(float(Residual) + float(branch) * float(Gate[..]))
-//   float      C = O(float(acc))
-// The library is compiled with -ffp-contract=off so none of these products and sums is
-// fused into an FMA: the FP32 rounding sequence is exactly the one written above.
+// W8A8 / FP8 / BF16 / FP16 linear layers on gfx950 MFMA: tile schedules and launches.  Epilogues in
+// gemm_epilogue.h, the small-tile kernels in gemm_ring.h and gemm_decode.h, the choice among all of
+// them in gemm_plan.h.
 #pragma once
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
 
-#include "gemm_core.h"
+#include "gemm_decode.h"
+#include "gemm_plan.h"
+#include "gemm_ring.h"
 
 namespace m5k {
 namespace gemm {
 namespace detail {
-
-enum { EPI_NONE = 0, EPI_VECTOR = 1, EPI_TABLE = 2 };
-
-struct EpiParams {
-  const float* sa;
-  const float* sb;
-  void* c;
-  const float* bias;
-  const int32_t* bias_map;
-  const uint16_t* residual;
-  const uint16_t* gate;
-  const int32_t* gate_map;
-  int coalesced;  // 16-bit output with N % 8 == 0 and 16-byte aligned c / residual / gate
-};
-
-// RAW: write INT32 accumulators (I8 only).
-// Wave grid used by every GEMM kernel of the library.
-using KernelGrid = Grid8;
-
-// The tile's scales ahead of the main loop (quantized modes with a scale epilogue; nothing for the
-// others).
-template <int MODE, bool RAW, class G>
-__device__ __forceinline__ TileScalePrefetch<G> prefetch_scales(const EpiParams& p, int M, int N, int m0, int n0) {
-  if constexpr ((MODE == I8 || MODE == F8) && !RAW) return TileScalePrefetch<G>(p.sa, p.sb, M, N, m0, n0);
-  else return TileScalePrefetch<G>(nullptr, nullptr, 0, 0, 0, 0);
-}
-
-// Scale epilogue of one 256 x G::TN tile (every thread of the workgroup calls it; the LDS is
-// free).  RAW writes the INT32 accumulators.  The per-row and per-column operands of the
-// lane's elements (scales, bias vector) are loaded in one batch before the arithmetic, and a
-// bias table's offsets and values one block row at a time, so the epilogue waits for memory a
-// few times instead of once per element.
-template <int MODE, int OUT_DT, int BIAS, int GATE, bool RAW, class G = KernelGrid>
-__device__ __forceinline__ void epilogue(const AccTile<MODE, G>& acc, int M, int N, int m0, int n0,
-                                         const EpiParams& p, const TileScalePrefetch<G>& pre) {
-  using Geo = AccGeom<MODE, G>;
-  constexpr bool QUANT = MODE == I8 || MODE == F8;
-  const int tid = tid_after_mainloop();
-  const Geo geo(tid);
-  if constexpr (RAW) {
-#pragma unroll
-    for (int i = 0; i < Geo::FM; ++i)
-#pragma unroll
-      for (int j = 0; j < Geo::FN; ++j)
-#pragma unroll
-        for (int e = 0; e < Geo::PER; ++e) {
-          const int m = m0 + geo.row(i, e), n = n0 + geo.col(j);
-          if (m < M && n < N) static_cast<int32_t*>(p.c)[(int64_t)m * N + n] = acc[i][j][e];
-        }
-    return;
-  } else {
-    float cs[QUANT ? Geo::FN : 1];
-    const float* sc = nullptr;
-    if constexpr (QUANT) {
-      const TileScales<G> ts(pre, tid);
-      sc = ts.s;
-#pragma unroll
-      for (int j = 0; j < Geo::FN; ++j) cs[j] = ts.col(geo.col(j));
-    }
-    float bvec[BIAS == EPI_VECTOR ? Geo::FN : 1];
-    if constexpr (BIAS == EPI_VECTOR) {
-#pragma unroll
-      for (int j = 0; j < Geo::FN; ++j) {
-        const int n = n0 + geo.col(j);
-        bvec[j] = n < N ? p.bias[n] : 0.0f;
-      }
-    }
-    // FP32 value of block row i's elements: the scale epilogue, then the bias (a bias table's
-    // row offsets and values are loaded per block row, two batches).
-    auto row_values = [&](int i, float (&val)[Geo::FN][Geo::PER]) {
-      float rs[QUANT ? Geo::PER : 1];
-      if constexpr (QUANT) {
-#pragma unroll
-        for (int e = 0; e < Geo::PER; ++e) rs[e] = sc[geo.row(i, e)];
-      }
-      float tb[BIAS == EPI_TABLE ? Geo::FN : 1][BIAS == EPI_TABLE ? Geo::PER : 1];
-      if constexpr (BIAS == EPI_TABLE) {
-        int64_t brow[Geo::PER];
-#pragma unroll
-        for (int e = 0; e < Geo::PER; ++e) {
-          const int m = m0 + geo.row(i, e);
-          brow[e] = m < M ? (int64_t)p.bias_map[m] * N : 0;
-        }
-#pragma unroll
-        for (int j = 0; j < Geo::FN; ++j)
-#pragma unroll
-          for (int e = 0; e < Geo::PER; ++e) {
-            const int m = m0 + geo.row(i, e), n = n0 + geo.col(j);
-            tb[j][e] = (m < M && n < N) ? p.bias[brow[e] + n] : 0.0f;
-          }
-      }
-#pragma unroll
-      for (int j = 0; j < Geo::FN; ++j)
-#pragma unroll
-        for (int e = 0; e < Geo::PER; ++e) {
-          float value;
-          if constexpr (QUANT) value = (static_cast<float>(acc[i][j][e]) * rs[e]) * cs[j];
-          else value = acc[i][j][e];
-          if constexpr (BIAS == EPI_VECTOR) value = value + bvec[j];
-          if constexpr (BIAS == EPI_TABLE) value = value + tb[j][e];
-          val[j][e] = value;
-        }
-    };
-
-    // 16-bit outputs: stage the rounded tile (the BF16 branch for the gated form) in the LDS the
-    // main loop has released, then write whole 512-byte tile rows with 16-byte streaming stores.
-    if constexpr (OUT_DT == M5K_BF16 || OUT_DT == M5K_F16) {
-      if (p.coalesced) {
-        uint16_t* tile = reinterpret_cast<uint16_t*>(g_lds);
-#pragma unroll
-        for (int i = 0; i < Geo::FM; ++i) {
-          float val[Geo::FN][Geo::PER];
-          row_values(i, val);
-#pragma unroll
-          for (int j = 0; j < Geo::FN; ++j)
-#pragma unroll
-            for (int e = 0; e < Geo::PER; ++e) {
-              // Entries past M or N are staged unmasked: the write-out below skips them.
-              const int r = geo.row(i, e), c = geo.col(j);
-              const float value = val[j][e];
-              tile[r * TILE16_STRIDE + c] = static_cast<uint16_t>(
-                  GATE != EPI_NONE || OUT_DT == M5K_BF16 ? f32_to_bf16_bits(value) : f32_to_f16_bits(value));
-            }
-        }
-        __syncthreads();
-        constexpr int CPR = G::TN / 8;  // 16-byte chunks per tile row
-        for (int c = threadIdx.x; c < BM * CPR; c += G::THREADS) {
-          const int r = c / CPR, cc = c % CPR;
-          const int m = m0 + r, n = n0 + 8 * cc;
-          if (m >= M || n >= N) continue;  // N % 8 == 0: a chunk is wholly in or out
-          uint4 w = *reinterpret_cast<const uint4*>(tile + r * TILE16_STRIDE + 8 * cc);
-          const int64_t idx = (int64_t)m * N + n;
-          if constexpr (GATE != EPI_NONE) {
-            const int64_t goff = GATE == EPI_TABLE ? (int64_t)p.gate_map[m] * N : 0;
-            const uint4 rw = *reinterpret_cast<const uint4*>(p.residual + idx);
-            const uint4 gw = *reinterpret_cast<const uint4*>(p.gate + goff + n);
-            const uint32_t bs[4] = {w.x, w.y, w.z, w.w}, rs[4] = {rw.x, rw.y, rw.z, rw.w},
-                           gs[4] = {gw.x, gw.y, gw.z, gw.w};
-            uint32_t out[4];
-#pragma unroll
-            for (int t = 0; t < 4; ++t) {
-              const float lo = bf16_bits_to_f32(rs[t] & 0xFFFFu) +
-                               bf16_bits_to_f32(bs[t] & 0xFFFFu) * bf16_bits_to_f32(gs[t] & 0xFFFFu);
-              const float hi =
-                  bf16_bits_to_f32(rs[t] >> 16) + bf16_bits_to_f32(bs[t] >> 16) * bf16_bits_to_f32(gs[t] >> 16);
-              out[t] = f32x2_to_bf16x2(lo, hi);
-            }
-            w = make_uint4(out[0], out[1], out[2], out[3]);
-          }
-          store_stream16(static_cast<uint16_t*>(p.c) + idx, w);
-        }
-        return;
-      }
-    }
-
-#pragma unroll
-    for (int i = 0; i < Geo::FM; ++i) {
-      float val[Geo::FN][Geo::PER];
-      row_values(i, val);
-      // The gated form's residual and gate values of this block row, loaded in one batch.
-      float res[GATE != EPI_NONE ? Geo::FN : 1][GATE != EPI_NONE ? Geo::PER : 1];
-      float gte[GATE != EPI_NONE ? Geo::FN : 1][GATE != EPI_NONE ? Geo::PER : 1];
-      if constexpr (GATE != EPI_NONE) {
-#pragma unroll
-        for (int j = 0; j < Geo::FN; ++j)
-#pragma unroll
-          for (int e = 0; e < Geo::PER; ++e) {
-            const int m = m0 + geo.row(i, e), n = n0 + geo.col(j);
-            const bool in = m < M && n < N;
-            const int64_t goff = GATE == EPI_TABLE && in ? (int64_t)p.gate_map[m] * N : 0;
-            res[j][e] = in ? bf16_bits_to_f32(p.residual[(int64_t)m * N + n]) : 0.0f;
-            gte[j][e] = in ? bf16_bits_to_f32(p.gate[goff + n]) : 0.0f;
-          }
-      }
-#pragma unroll
-      for (int j = 0; j < Geo::FN; ++j)
-#pragma unroll
-        for (int e = 0; e < Geo::PER; ++e) {
-          const int m = m0 + geo.row(i, e), n = n0 + geo.col(j);
-          if (m >= M || n >= N) continue;
-          const int64_t idx = (int64_t)m * N + n;
-          if constexpr (GATE != EPI_NONE) {
-            const float branch = round_through<M5K_BF16>(val[j][e]);
-            store_elem<M5K_BF16>(p.c, idx, res[j][e] + branch * gte[j][e]);
-          } else {
-            store_elem<OUT_DT>(p.c, idx, val[j][e]);
-          }
-        }
-    }
-  }
-}
 
 // One 256 x G::TN output tile per workgroup.
 template <int MODE, bool ALIGNED, int OUT_DT, int BIAS, int GATE, bool RAW, class G = KernelGrid>
@@ -391,6 +195,88 @@ inline int plan_schedule(bool md16, bool i8, int64_t m, int64_t n, int cus, int6
   return full >= 0 ? SCHED_MIXED : SCHED_PLAIN;
 }
 
+// ---- Small tiles (gemm_ring.h, gemm_decode.h) ----------------------------------------------------
+
+// Ring shapes by tile.  64 KiB of stages let two 64 x 64 workgroups share a CU; 96 KiB ("deep") keep
+// one, with twice the K per barrier.  FP8 stages hold two planes, so half as many.
+template <int MODE>
+struct RingTiles {
+  using T128 = ring::Cfg<MODE, 128, 128, MODE == F8 ? 2 : 4>;
+  using T64 = ring::Cfg<MODE, 64, 64, MODE == F8 ? 2 : 4>;
+  using Deep = ring::Cfg<MODE, 64, 64, 3, 2>;
+  // Unaligned operands: two stage buffers, filled through registers.
+  using U128 = ring::Cfg<MODE, 128, 128, 2, 1>;
+  using U64 = ring::Cfg<MODE, 64, 64, 2, 1>;
+};
+
+constexpr bool small_mode(int mode) { return mode == I8 || mode == F8 || mode == BF16 || mode == F16; }
+
+// Time of the 256-row schedules' launch in 256 x 256 tile times.
+inline double units_256(bool md16, int64_t m, int64_t n, int cus) {
+  const int64_t tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN);
+  if (cus <= 0) return static_cast<double>(tiles);
+  const int64_t full = mixed_full_tiles(m, n, cus);
+  if (md16 && narrow_pays(m, n, cus, full)) {
+    const int64_t narrow = ((m + BM - 1) / BM) * ((n + Grid8Narrow::TN - 1) / Grid8Narrow::TN);
+    return static_cast<double>((narrow + cus - 1) / cus) * kNarrowTileCost;
+  }
+  if (full >= 0) return 1.03 * mixed_makespan(full, 2 * (tiles - full), cus);
+  return static_cast<double>((tiles + cus - 1) / cus);
+}
+
+// The tile of an [m, n] output with rows of kb bytes (no partial sums): one of gemm_plan.h's, or
+// TILE_256 for the 256-row schedules.  Aligned operands under a forced schedule run that schedule.
+// Float rows of under 1 KiB stay there too: the smaller tiles split K over waves, and eight 128-byte
+// lines leave each of them one or none.  FP8's unaligned operands keep the register-staged loop.
+inline plan::Choice plan_tile(int mode, int64_t m, int64_t n, int64_t kb, int cus, bool aligned, int max_splits = 1,
+                              double limit_us = 1e30) {
+  const plan::Choice none{plan::TILE_256, 1, 0.0};
+  const bool md16 = mode == I8 || mode == BF16 || mode == F16;
+  if (!small_mode(mode) || cus <= 0 || (!aligned && mode == F8)) return none;
+  if (aligned) {
+    int64_t full = -1;
+    if (forced_schedule(md16, mode == I8, m, n, cus, full) >= 0) return none;
+    if (mode != I8 && kb < 8 * BKB) return none;
+    limit_us = std::min(limit_us, plan::tile256_us(units_256(md16, m, n, cus), n, kb));
+  }
+  return plan::choose(m, n, kb, cus, aligned, max_splits, limit_us);
+}
+
+template <class C, bool ALIGNED, int OUT_DT, int BIAS, int GATE>
+int launch_ring(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int64_t kb, const EpiParams& q,
+                hipStream_t st, const char* name) {
+  const int64_t wgs = ((m + C::TM - 1) / C::TM) * ((n + C::TN - 1) / C::TN);
+  M5K_REQUIRE(wgs <= 0x7FFFFFFF, "%s: too many tiles", name);
+  launch_kernel(ring::gemm_ring_kernel<C, ALIGNED, OUT_DT, BIAS, GATE>, dim3(static_cast<unsigned>(wgs)), dim3(512), st,
+                A, B, (int)m, (int)n, kb, q);
+  return launch_status(name);
+}
+
+template <int MODE, int OUT_DT, int BIAS, int GATE>
+int launch_small(int tile, bool aligned, const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int64_t kb,
+                 const EpiParams& q, hipStream_t st, const char* name) {
+  using R = RingTiles<MODE>;
+  if constexpr (MODE != F8) {
+    if (!aligned)
+      return tile == plan::TILE_128
+                 ? launch_ring<typename R::U128, false, OUT_DT, BIAS, GATE>(A, B, m, n, kb, q, st, name)
+                 : launch_ring<typename R::U64, false, OUT_DT, BIAS, GATE>(A, B, m, n, kb, q, st, name);
+  }
+  switch (tile) {
+    case plan::TILE_128: return launch_ring<typename R::T128, true, OUT_DT, BIAS, GATE>(A, B, m, n, kb, q, st, name);
+    case plan::TILE_64: return launch_ring<typename R::T64, true, OUT_DT, BIAS, GATE>(A, B, m, n, kb, q, st, name);
+    case plan::TILE_64_DEEP:
+      return launch_ring<typename R::Deep, true, OUT_DT, BIAS, GATE>(A, B, m, n, kb, q, st, name);
+    default: break;
+  }
+  const dim3 wgs(static_cast<unsigned>((n + 15) / 16)), block(64 * decode::WAVES);
+  if (m <= 16)
+    launch_kernel(decode::gemm_decode_kernel<MODE, 1, OUT_DT, BIAS, GATE>, wgs, block, st, A, B, (int)m, (int)n, kb, q);
+  else
+    launch_kernel(decode::gemm_decode_kernel<MODE, 2, OUT_DT, BIAS, GATE>, wgs, block, st, A, B, (int)m, (int)n, kb, q);
+  return launch_status(name);
+}
+
 template <int MODE, int OUT_DT, int BIAS, int GATE, bool RAW>
 int launch(const void* a, const void* b, int64_t m, int64_t n, int64_t k, const EpiParams& p,
            hipStream_t st, const char* name) {
@@ -404,6 +290,11 @@ int launch(const void* a, const void* b, int64_t m, int64_t n, int64_t k, const 
   auto* B = static_cast<const uint8_t*>(b);
   EpiParams q = p;
   q.coalesced = n % 8 == 0 && aligned16(p.c) && (p.residual == nullptr || (aligned16(p.residual) && aligned16(p.gate)));
+  if constexpr (small_mode(MODE) && !RAW) {
+    const plan::Choice small = plan_tile(MODE, m, n, kb, device_cus(), aligned);
+    if (small.tile != plan::TILE_256)
+      return launch_small<MODE, OUT_DT, BIAS, GATE>(small.tile, aligned, A, B, m, n, kb, q, st, name);
+  }
   if (aligned) {
     int64_t full = -1;
     // The narrow 256 x 224 tile serves the 16 x 16 modes with 16-byte fragments (INT8, BF16,
@@ -433,8 +324,11 @@ int launch(const void* a, const void* b, int64_t m, int64_t n, int64_t k, const 
     } else {
       launch_kernel(gemm_kernel<MODE, true, OUT_DT, BIAS, GATE, RAW>, grid, block, st, A, B, (int)m, (int)n, kb, q);
     }
-  } else
+  } else if constexpr (RAW || MODE == F8 || MODE == F32) {
     launch_kernel(gemm_kernel<MODE, false, OUT_DT, BIAS, GATE, RAW>, grid, block, st, A, B, (int)m, (int)n, kb, q);
+  } else {
+    return launch_small<MODE, OUT_DT, BIAS, GATE>(plan::TILE_64, false, A, B, m, n, kb, q, st, name);
+  }
   return launch_status(name);
 }
 
@@ -468,108 +362,140 @@ __global__ __launch_bounds__(G::THREADS, 1) void gemm_splitk_kernel(const uint8_
   });
 }
 
-template <int OUT_DT, int BIAS, int GATE, class P = int32_t>
+// Sums the partial tiles in split order and applies the epilogue.  VEC = 4: four consecutive columns
+// per thread (N % 4 == 0 and 16-byte aligned c), one 16-byte load per split and one packed store; the
+// splits' loads do not depend on each other, so a thread has them all in flight.
+template <int OUT_DT, int BIAS, int GATE, class P, int VEC>
 __global__ __launch_bounds__(256) void splitk_epilogue_kernel(const P* __restrict__ partial, int splits, int M, int N,
                                                               EpiParams p) {
+  constexpr int MODE = std::is_same<P, float>::value ? F8 : I8;
   const int64_t total = static_cast<int64_t>(M) * N;
-  for (int64_t idx = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; idx < total;
-       idx += static_cast<int64_t>(gridDim.x) * 256) {
-    P v = 0;
-    for (int s = 0; s < splits; ++s) v += partial[s * total + idx];
+  for (int64_t idx = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * VEC; idx < total;
+       idx += static_cast<int64_t>(gridDim.x) * 256 * VEC) {
     const int m = static_cast<int>(idx / N), n = static_cast<int>(idx - static_cast<int64_t>(m) * N);
-    float value = (static_cast<float>(v) * p.sa[m]) * p.sb[n];
-    if constexpr (BIAS != EPI_NONE) {
-      const int64_t boff = BIAS == EPI_TABLE ? (int64_t)p.bias_map[m] * N : 0;
-      value = value + p.bias[boff + n];
-    }
-    if constexpr (GATE != EPI_NONE) {
-      const int64_t goff = GATE == EPI_TABLE ? (int64_t)p.gate_map[m] * N : 0;
-      const float branch = round_through<M5K_BF16>(value);
-      const float res = bf16_bits_to_f32(p.residual[idx]);
-      const float g = bf16_bits_to_f32(p.gate[goff + n]);
-      store_elem<M5K_BF16>(p.c, idx, res + branch * g);
+    if constexpr (VEC == 1) {
+      P v = 0;
+      for (int s = 0; s < splits; ++s) v += partial[s * total + idx];
+      store_elem<OUT_DT>(p.c, idx, result_value<MODE, BIAS, GATE>(p, v, m, n, N));
     } else {
-      store_elem<OUT_DT>(p.c, idx, value);
+      typedef P vec4 __attribute__((ext_vector_type(4)));
+      vec4 v = {0, 0, 0, 0};
+#pragma unroll 4
+      for (int s = 0; s < splits; ++s) v += *reinterpret_cast<const vec4*>(partial + s * total + idx);
+      float r[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) r[e] = result_value<MODE, BIAS, GATE>(p, v[e], m, n + e, N);
+      if constexpr (OUT_DT == M5K_F32) {
+        *reinterpret_cast<float4*>(static_cast<float*>(p.c) + idx) = make_float4(r[0], r[1], r[2], r[3]);
+      } else {
+        uint2 w;
+        if constexpr (OUT_DT == M5K_BF16) w = make_uint2(f32x2_to_bf16x2(r[0], r[1]), f32x2_to_bf16x2(r[2], r[3]));
+        else
+          w = make_uint2(f32_to_f16_bits(r[0]) | (f32_to_f16_bits(r[1]) << 16),
+                         f32_to_f16_bits(r[2]) | (f32_to_f16_bits(r[3]) << 16));
+        *reinterpret_cast<uint2*>(static_cast<uint16_t*>(p.c) + idx) = w;
+      }
     }
   }
 }
 
-template <int OUT_DT, int BIAS, int GATE>
-int launch_splitk(const int8_t* a, const int8_t* b, int64_t m, int64_t n, int64_t k, const EpiParams& p,
-                  int splits, int32_t* workspace, hipStream_t st, const char* name) {
-  const int64_t kt_total = k_stages(k);
-  const int64_t per = (kt_total + splits - 1) / splits;
-  const int used = static_cast<int>((kt_total + per - 1) / per);  // no empty split
-  // 256 x 64 tiles (K <= 8192) or 256 x 128 tiles when their workgroups fit in one round, so
-  // a few K ranges fill the chip and the INT32 partials (splits x M x N) stay small next to the
-  // weights streamed.  Measured against 256 x 256 tiles with the split count sized to each:
-  // 256 x 64 1.4-1.6x faster at K 4096-5376 (M 1-256), equal at K 16384 and 5% slower at K
-  // 14336, hence its K limit; 256 x 128 1.15-1.23x faster where 256 x 64 does not fit (N 14336,
-  // or K 14336-16384); at M 384-1024 the narrower tiles were 1.1-1.45x faster.
-  const int cus = device_cus();
-  auto fits = [&](int width) {
-    return cus > 0 && ((m + BM - 1) / BM) * ((n + width - 1) / width) * used <= static_cast<int64_t>(cus);
-  };
-  const int tn = k <= 8192 && fits(Grid8Skinny::TN) ? Grid8Skinny::TN : fits(HalfGrid::TN) ? HalfGrid::TN : BN;
-  const int64_t tiles = ((m + BM - 1) / BM) * ((n + tn - 1) / tn);
-  M5K_REQUIRE(tiles * used <= 0x7FFFFFFF, "%s: too many workgroups", name);
-  const dim3 wgs(static_cast<unsigned>(tiles * used)), block(KernelGrid::THREADS);
-  auto* A = reinterpret_cast<const uint8_t*>(a);
-  auto* B = reinterpret_cast<const uint8_t*>(b);
-  if (tn == Grid8Skinny::TN)
-    gemm_splitk_kernel<I8, Grid8Skinny><<<wgs, block, 0, st>>>(A, B, (int)m, (int)n, k, used, per, workspace);
-  else if (tn == HalfGrid::TN)
-    gemm_splitk_kernel<I8, HalfGrid><<<wgs, block, 0, st>>>(A, B, (int)m, (int)n, k, used, per, workspace);
+template <int OUT_DT, int BIAS, int GATE, class P>
+int launch_splitk_epilogue(const P* workspace, int used, int64_t m, int64_t n, const EpiParams& p, hipStream_t st,
+                           const char* name) {
+  const bool vec = n % 4 == 0 && aligned16(p.c) && aligned16(workspace);
+  const int64_t blocks = (m * n / (vec ? 4 : 1) + 255) / 256;
+  const dim3 grid(static_cast<unsigned>(blocks < 65536 ? blocks : 65536));
+  if (vec)
+    launch_kernel(splitk_epilogue_kernel<OUT_DT, BIAS, GATE, P, 4>, grid, dim3(256), st, workspace, used, (int)m, (int)n, p);
   else
-    gemm_splitk_kernel<I8><<<wgs, block, 0, st>>>(A, B, (int)m, (int)n, k, used, per, workspace);
-  if (int rc = launch_status(name)) return rc;
-  const int64_t blocks = (m * n + 255) / 256;
-  const unsigned grid = static_cast<unsigned>(blocks < 65536 ? blocks : 65536);
-  splitk_epilogue_kernel<OUT_DT, BIAS, GATE><<<dim3(grid), dim3(256), 0, st>>>(workspace, used, (int)m, (int)n, p);
+    launch_kernel(splitk_epilogue_kernel<OUT_DT, BIAS, GATE, P, 1>, grid, dim3(256), st, workspace, used, (int)m, (int)n, p);
   return launch_status(name);
+}
+
+template <class C, class P>
+int launch_ring_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int64_t kb, int splits, P* workspace,
+                       int& used, hipStream_t st, const char* name) {
+  const int64_t total = ring::stages<C>(kb);
+  const int64_t per = (total + splits - 1) / splits;
+  used = static_cast<int>((total + per - 1) / per);  // no empty split
+  const int64_t wgs = ((m + C::TM - 1) / C::TM) * ((n + C::TN - 1) / C::TN) * used;
+  M5K_REQUIRE(wgs <= 0x7FFFFFFF, "%s: too many workgroups", name);
+  launch_kernel(ring::gemm_ring_splitk_kernel<C, P>, dim3(static_cast<unsigned>(wgs)), dim3(512), st, A, B, (int)m, (int)n,
+                kb, used, per, workspace);
+  return launch_status(name);
+}
+
+// At most `splits` K ranges per tile, as many as the planner expects to pay: a tile small enough to
+// fill the CUs needs none, and then no partial sums exist (128 x 4096 x 4096 INT8 with 4 ranges of 256
+// x 64 tiles and the epilogue pass 16.2 us; unsplit 64 x 64 tiles 9.7 us).  The 256-row tiles serve
+// what is left, middle M with a long K: 256 x 128 where their workgroups fit in one round, else 256 x
+// 256 (M 1024, N 5376, K 14336: 84 us with 3 ranges, 94 us unsplit).
+template <int MODE, int OUT_DT, int BIAS, int GATE, class P>
+int launch_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int64_t kb, const EpiParams& p, int splits,
+                  P* workspace, hipStream_t st, const char* name) {
+  constexpr bool md16 = MODE != F8;  // the narrow schedule's modes
+  const int64_t kt_total = k_stages(kb);
+  const int64_t per = (kt_total + splits - 1) / splits;
+  int used = static_cast<int>((kt_total + per - 1) / per);  // no empty split
+  const int cus = device_cus();
+  const int64_t tiles_m = (m + BM - 1) / BM;
+  const bool half = cus > 0 && tiles_m * ((n + HalfGrid::TN - 1) / HalfGrid::TN) * used <= static_cast<int64_t>(cus);
+  const int tn = half ? HalfGrid::TN : BN;
+  const int64_t wgs_256 = tiles_m * ((n + tn - 1) / tn) * used;
+  const double rounds = cus > 0 ? static_cast<double>((wgs_256 + cus - 1) / cus) : 1.0;
+  // Half tiles run short of their share here: 512 x 7168 x 14336 in 2 ranges 82 us, 768 x 5376 x 14336
+  // 69 us, where their time in a mixed launch predicts 62 and 64.
+  const double split_256 = plan::tile256_us(rounds * (half ? 1.25 * kHalfTileCost : 1.0), n, kb / used) +
+                           plan::split_us(m, n, used);
+  const double plain_256 = plan::tile256_us(units_256(md16, m, n, cus), n, kb);
+  const plan::Choice c = plan_tile(MODE, m, n, kb, cus, true, splits, std::min(split_256, plain_256));
+  if ((c.tile == plan::TILE_256 && plain_256 < split_256) || (c.tile != plan::TILE_256 && c.splits == 1))
+    return launch<MODE, OUT_DT, BIAS, GATE, false>(A, B, m, n, kb / Traits<MODE>::elem_bytes, p, st, name);
+  using R = RingTiles<MODE>;
+  int rc = M5K_OK;
+  if (c.tile == plan::TILE_128) {
+    rc = launch_ring_splitk<typename R::T128>(A, B, m, n, kb, c.splits, workspace, used, st, name);
+  } else if (c.tile == plan::TILE_64) {
+    rc = launch_ring_splitk<typename R::T64>(A, B, m, n, kb, c.splits, workspace, used, st, name);
+  } else if (c.tile == plan::TILE_64_DEEP) {
+    rc = launch_ring_splitk<typename R::Deep>(A, B, m, n, kb, c.splits, workspace, used, st, name);
+  } else {
+    M5K_REQUIRE(wgs_256 <= 0x7FFFFFFF, "%s: too many workgroups", name);
+    const dim3 wgs(static_cast<unsigned>(wgs_256)), block(KernelGrid::THREADS);
+    if (half)
+      launch_kernel(gemm_splitk_kernel<MODE, HalfGrid, P>, wgs, block, st, A, B, (int)m, (int)n, kb, used, per, workspace);
+    else
+      launch_kernel(gemm_splitk_kernel<MODE, KernelGrid, P>, wgs, block, st, A, B, (int)m, (int)n, kb, used, per, workspace);
+    rc = launch_status(name);
+  }
+  if (rc) return rc;
+  return launch_splitk_epilogue<OUT_DT, BIAS, GATE, P>(workspace, used, m, n, p, st, name);
 }
 
 template <int OUT_DT>
 int launch_i8_splitk(const int8_t* a, const int8_t* b, int64_t m, int64_t n, int64_t k, const EpiParams& p,
                      int splits, int32_t* workspace, hipStream_t st, const char* name) {
+  auto* A = reinterpret_cast<const uint8_t*>(a);
+  auto* B = reinterpret_cast<const uint8_t*>(b);
   if (p.bias) {
-    return p.bias_map ? launch_splitk<OUT_DT, EPI_TABLE, EPI_NONE>(a, b, m, n, k, p, splits, workspace, st, name)
-                      : launch_splitk<OUT_DT, EPI_VECTOR, EPI_NONE>(a, b, m, n, k, p, splits, workspace, st, name);
+    return p.bias_map ? launch_splitk<I8, OUT_DT, EPI_TABLE, EPI_NONE>(A, B, m, n, k, p, splits, workspace, st, name)
+                      : launch_splitk<I8, OUT_DT, EPI_VECTOR, EPI_NONE>(A, B, m, n, k, p, splits, workspace, st, name);
   }
   if (p.residual) {
-    return p.gate_map ? launch_splitk<M5K_BF16, EPI_NONE, EPI_TABLE>(a, b, m, n, k, p, splits, workspace, st, name)
-                      : launch_splitk<M5K_BF16, EPI_NONE, EPI_VECTOR>(a, b, m, n, k, p, splits, workspace, st, name);
+    return p.gate_map
+               ? launch_splitk<I8, M5K_BF16, EPI_NONE, EPI_TABLE>(A, B, m, n, k, p, splits, workspace, st, name)
+               : launch_splitk<I8, M5K_BF16, EPI_NONE, EPI_VECTOR>(A, B, m, n, k, p, splits, workspace, st, name);
   }
-  return launch_splitk<OUT_DT, EPI_NONE, EPI_NONE>(a, b, m, n, k, p, splits, workspace, st, name);
+  return launch_splitk<I8, OUT_DT, EPI_NONE, EPI_NONE>(A, B, m, n, k, p, splits, workspace, st, name);
 }
 
-// FP8 split-K: FP32 partial tiles, summed in split order by the same epilogue kernel.  The
-// 256 x 64 tile's waves hold two 16-row blocks, fewer than FP8's stage schedule takes, so the
-// split tiles are 256 x 128 where their workgroups fit in one round, else 256 x 256.  Each K
+// FP8 split-K: FP32 partial tiles, summed in split order by the same epilogue kernel.  Each K
 // range is its own FP32 accumulation, so the output can differ from the unsplit launch in the
 // last bits of the FP32 sum (FP8's accumulation order is not pinned); it is deterministic.
 template <int OUT_DT>
 int launch_f8_splitk(const uint8_t* a, const uint8_t* b, int64_t m, int64_t n, int64_t k, const EpiParams& p,
                      int splits, float* workspace, hipStream_t st, const char* name) {
-  const int64_t kt_total = k_stages(k);
-  const int64_t per = (kt_total + splits - 1) / splits;
-  const int used = static_cast<int>((kt_total + per - 1) / per);  // no empty split
-  const int cus = device_cus();
-  const bool half = cus > 0 && ((m + BM - 1) / BM) * ((n + HalfGrid::TN - 1) / HalfGrid::TN) * used <= cus;
-  const int tn = half ? HalfGrid::TN : BN;
-  const int64_t tiles = ((m + BM - 1) / BM) * ((n + tn - 1) / tn);
-  M5K_REQUIRE(tiles * used <= 0x7FFFFFFF, "%s: too many workgroups", name);
-  const dim3 wgs(static_cast<unsigned>(tiles * used)), block(KernelGrid::THREADS);
-  if (half)
-    gemm_splitk_kernel<F8, HalfGrid, float><<<wgs, block, 0, st>>>(a, b, (int)m, (int)n, k, used, per, workspace);
-  else
-    gemm_splitk_kernel<F8, KernelGrid, float><<<wgs, block, 0, st>>>(a, b, (int)m, (int)n, k, used, per, workspace);
-  if (int rc = launch_status(name)) return rc;
-  const int64_t blocks = (m * n + 255) / 256;
-  const unsigned grid = static_cast<unsigned>(blocks < 65536 ? blocks : 65536);
-  splitk_epilogue_kernel<OUT_DT, EPI_NONE, EPI_NONE, float>
-      <<<dim3(grid), dim3(256), 0, st>>>(workspace, used, (int)m, (int)n, p);
-  return launch_status(name);
+  return launch_splitk<F8, OUT_DT, EPI_NONE, EPI_NONE>(a, b, m, n, k, p, splits, workspace, st, name);
 }
 
 inline int check_shape(int64_t m, int64_t n, int64_t k, const char* name) {

@@ -230,12 +230,13 @@ __device__ __forceinline__ uint4 norm_rope_fast(const float (&z)[8], const LaneR
   return rope_apply<HALF8>(z, r, cw, sw, head_inv(head_sumsq(z), eps));
 }
 
-// Epilogue of one 256 x G::TN projection tile (G::TN = 256: two heads, or 128: one head), called
+// Epilogue of one G::TM x G::TN projection tile (G::TN = 256: two heads, or 128: one head), called
 // by every thread after the main loop: the BF16 projection is staged in the LDS the loop has
 // released, then 16-lane groups normalize and rotate (row, head) pairs.
 template <int MODE, class G>
 __device__ __forceinline__ void qk_tile_epilogue(const AccTile<MODE, G>& acc, int M, int N, int m0, int n0,
-                                                 const TileScalePrefetch<G>& pre, const QkParams& p, int fast) {
+                                                 const TileScalePrefetch<G>& pre, const QkParams& p, int fast,
+                                                 uint8_t* lds = g_lds) {
   static_assert(G::TN % HEAD == 0, "projection tiles hold whole heads");
   constexpr int HPT = G::TN / HEAD;  // heads per tile
   // Everything the epilogue loads depends on the lane index taken here, after the main loop,
@@ -245,19 +246,20 @@ __device__ __forceinline__ void qk_tile_epilogue(const AccTile<MODE, G>& acc, in
   __asm__ volatile("" : "+v"(tid_after));
   const int group = tid_after >> 4, lg = tid_after & 15;
   constexpr int GROUPS = G::THREADS / 16;  // 32 groups of 16 lanes
-  constexpr int ROWS_PER_GROUP = BM / GROUPS;
+  constexpr int ROWS_PER_GROUP = G::TM / GROUPS;
   const int heads_here = min(G::TN, N - n0) / HEAD;  // N is a multiple of 128
 
-  // BF16 projection tile [256 rows][G::TN cols] in LDS (row stride TILE16_STRIDE).  The main
+  // BF16 projection tile [G::TM rows][G::TN cols] in LDS (row stride STRIDE).  The main
   // loop ended with a drained DMA and a barrier, so the stage ring is free.
-  uint16_t* tile = reinterpret_cast<uint16_t*>(g_lds);
+  constexpr int STRIDE = EpiLayout<G>::STRIDE;
+  uint16_t* tile = reinterpret_cast<uint16_t*>(lds);
   {
     using Geo = AccGeom<MODE, G>;
     const Geo geo(tid_after);
     float cs[Geo::FN];
     const float* sc = nullptr;
     if constexpr (MODE == I8) {
-      const TileScales<G> ts(pre, tid_after);
+      const TileScales<G> ts(pre, tid_after, lds);
       sc = ts.s;
 #pragma unroll
       for (int j = 0; j < Geo::FN; ++j) cs[j] = ts.col(geo.col(j));
@@ -278,7 +280,7 @@ __device__ __forceinline__ void qk_tile_epilogue(const AccTile<MODE, G>& acc, in
           float value;
           if constexpr (MODE == I8) value = (static_cast<float>(acc[i][j][e]) * rs[e]) * cs[j];
           else value = acc[i][j][e];
-          tile[r * TILE16_STRIDE + c] = static_cast<uint16_t>(f32_to_bf16_bits(value));
+          tile[r * STRIDE + c] = static_cast<uint16_t>(f32_to_bf16_bits(value));
         }
     }
   }
@@ -289,7 +291,7 @@ __device__ __forceinline__ void qk_tile_epilogue(const AccTile<MODE, G>& acc, in
   // words spilled 35 VGPRs to scratch; this form uses 228 VGPRs and no scratch, same bits (C5
   // fused projection 162.6 -> 160.2 us, one box).
   LaneRope lr, lrk;  // Q (or single-projection) gamma; K gamma in the grouped layout
-  constexpr int LOOKAHEAD = 4;  // rows of cos/sin in flight ahead of the row being rotated
+  constexpr int LOOKAHEAD = ROWS_PER_GROUP < 4 ? ROWS_PER_GROUP : 4;  // rows of cos/sin in flight ahead of the row being rotated
   uint4 cw[ROWS_PER_GROUP], sw[ROWS_PER_GROUP];
   int row0 = m0 + group;
   __asm__ volatile("" : "+v"(row0));
@@ -314,7 +316,7 @@ __device__ __forceinline__ void qk_tile_epilogue(const AccTile<MODE, G>& acc, in
     constexpr int PAIRS = ROWS_PER_GROUP * HPT;
     static_assert(PAIRS <= 16, "one (row, head) pair per lane of the group");
     auto pair_words = [&](int i, int h) {
-      return *reinterpret_cast<const uint4*>(tile + (group + GROUPS * i) * TILE16_STRIDE + h * HEAD + 8 * lg);
+      return *reinterpret_cast<const uint4*>(tile + (group + GROUPS * i) * STRIDE + h * HEAD + 8 * lg);
     };
     float ss_mine = 0.0f;
 #pragma unroll
@@ -356,12 +358,12 @@ __device__ __forceinline__ void qk_tile_epilogue(const AccTile<MODE, G>& acc, in
     }
     return;
   }
-  for (int q = group; q < BM * HPT; q += GROUPS) {
+  for (int q = group; q < G::TM * HPT; q += GROUPS) {
     const int local_row = q / HPT, local_head = q % HPT;
     const int row = m0 + local_row;
     const int block = n0 / HEAD + local_head;
     if (row >= M || block * HEAD >= N) continue;  // uniform across the 16-lane group
-    const uint16_t* src = tile + local_row * TILE16_STRIDE + local_head * HEAD;
+    const uint16_t* src = tile + local_row * STRIDE + local_head * HEAD;
     const BlockDst d = block_dst(p, block);
     if (d.gamma == nullptr) {
       store_stream16(d.out + (static_cast<int64_t>(d.head) * M + row) * HEAD + 8 * lg,
@@ -386,7 +388,7 @@ __device__ __forceinline__ TileScalePrefetch<G> qk_prefetch_scales(const float* 
   else return TileScalePrefetch<G>(nullptr, nullptr, 0, 0, 0, 0);
 }
 
-template <int MODE, bool ALIGNED>
+template <int MODE>
 __global__ __launch_bounds__(KernelGrid::THREADS, 1) void qk_fused_kernel(const uint8_t* __restrict__ A,
                                                                           const uint8_t* __restrict__ B, int M, int N,
                                                                           int64_t Kb, const float* __restrict__ sa,
@@ -399,9 +401,31 @@ __global__ __launch_bounds__(KernelGrid::THREADS, 1) void qk_fused_kernel(const 
   const int m0 = tm * BM, n0 = tn * BN;
   const TileScalePrefetch<G> pre = qk_prefetch_scales<MODE, G>(sa, sb, M, N, m0, n0);
   AccTile<MODE, G> acc;
-  if constexpr (ALIGNED) mainloop_dma<MODE, G>(A, B, M, N, Kb, m0, n0, acc, 0, k_stages(Kb));
-  else mainloop_staged<MODE, G>(A, B, M, N, Kb, m0, n0, acc);
+  mainloop_dma<MODE, G>(A, B, M, N, Kb, m0, n0, acc, 0, k_stages(Kb));
   qk_tile_epilogue<MODE, G>(acc, M, N, m0, n0, pre, p, fast);
+}
+
+// Short and middle M, and unaligned operands: the ring GEMM's 128 x 128 tile, one head wide.  An
+// output of few 256 x 256 tiles leaves CUs idle in the kernels above (M 128, 56 heads of grouped Q/K/V,
+// K 5376, INT8: 50.7 us; 168 tiles of one head here: 33 us).
+template <class C, bool ALIGNED>
+__global__ __launch_bounds__(512, 1) void qk_ring_kernel(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
+                                                         int M, int N, int64_t Kb, const float* __restrict__ sa,
+                                                         const float* __restrict__ sb, QkParams p, int fast) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[C::LDS];
+  using G = typename C::G;
+  static_assert(C::TN == HEAD, "one head per tile");
+  const int tiles_m = (M + C::TM - 1) / C::TM, tiles_n = N / HEAD;
+  int tm, tn;
+  tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int m0 = tm * C::TM, n0 = tn * HEAD;
+  const TileScalePrefetch<G> pre = qk_prefetch_scales<C::MODE, G>(sa, sb, M, N, m0, n0);
+  ring::Acc<C> acc;
+  if constexpr (ALIGNED) ring::mainloop<C>(A, B, M, N, Kb, m0, n0, acc, 0, ring::stages<C>(Kb), lds);
+  else ring::mainloop_unaligned<C>(A, B, M, N, Kb, m0, n0, acc, lds);
+  ring::HalfAcc<C> half;
+  ring::exchange<C>(acc, half, lds, threadIdx.x >> 6, threadIdx.x & 63);
+  qk_tile_epilogue<C::MODE, G>(half, M, N, m0, n0, pre, p, fast, lds);
 }
 
 // The mixed schedule of the GEMM library (gemm_mixed_kernel) for the fused projection: the
@@ -441,29 +465,39 @@ __global__ __launch_bounds__(KernelGrid::THREADS, 1) void qk_mixed_kernel(const 
   }
 }
 
-// Staged postprocess of a BF16 [M, N] projection: one 16-lane group per (row, head), consecutive
-// groups walking the heads of a row (coalesced 256-byte reads).
+// Staged postprocess of a BF16 [M, N] projection: one 16-lane group per (row, 128-column block),
+// consecutive groups walking the blocks of a row (coalesced 256-byte reads).  V blocks of the grouped
+// layout are copied.
 __global__ __launch_bounds__(256) void qk_norm_rope_kernel(const uint16_t* __restrict__ P, int64_t M, int64_t N,
                                                            QkParams p, int fast) {
-  const int64_t heads = N / HEAD;
+  const int64_t blocks = N / HEAD;
   const int64_t q = static_cast<int64_t>(blockIdx.x) * 16 + (threadIdx.x >> 4);
   const int lg = threadIdx.x & 15;
-  if (q >= M * heads) return;  // whole 16-lane groups leave together
-  const int64_t row = q / heads;
-  const int head = static_cast<int>(q - row * heads);
-  const uint16_t* src = P + row * N + static_cast<int64_t>(head) * HEAD;
-  float z[8];
-  unpack8_bf16(*reinterpret_cast<const uint4*>(src + 8 * lg), z);
-  if (fast) {
-    const LaneRope lr = lane_rope(p, p.gamma, lg);
-    uint4 cw, sw;
-    lane_cos_sin(p, lr, row, lg, cw, sw);
-    const uint4 out = p.rope_half == 64 ? norm_rope_fast<true>(z, lr, cw, sw, p.eps)
-                                        : norm_rope_fast<false>(z, lr, cw, sw, p.eps);
-    store_stream16(p.y + (static_cast<int64_t>(head) * M + row) * HEAD + 8 * lg, out);
+  if (q >= M * blocks) return;  // whole 16-lane groups leave together
+  const int64_t row = q / blocks;
+  const int block = static_cast<int>(q - row * blocks);
+  const uint16_t* src = P + row * N + static_cast<int64_t>(block) * HEAD;
+  const BlockDst d = block_dst(p, block);
+  const uint4 w = *reinterpret_cast<const uint4*>(src + 8 * lg);
+  uint16_t* dst = d.out + (static_cast<int64_t>(d.head) * M + row) * HEAD + 8 * lg;
+  if (d.gamma == nullptr) {
+    store_stream16(dst, w);
     return;
   }
-  norm_rope_16(z, [&](int d) { return bf16_bits_to_f32(src[d]); }, p, row, M, head, lg);
+  float z[8];
+  unpack8_bf16(w, z);
+  if (fast) {
+    const LaneRope lr = lane_rope(p, d.gamma, lg);
+    uint4 cw, sw;
+    lane_cos_sin(p, lr, row, lg, cw, sw);
+    store_stream16(dst, p.rope_half == 64 ? norm_rope_fast<true>(z, lr, cw, sw, p.eps)
+                                          : norm_rope_fast<false>(z, lr, cw, sw, p.eps));
+    return;
+  }
+  QkParams ps = p;
+  ps.gamma = d.gamma;
+  ps.y = d.out;
+  norm_rope_16(z, [&](int c) { return bf16_bits_to_f32(src[c]); }, ps, row, M, d.head, lg);
 }
 
 // The fast path needs whole 8-channel lanes per RoPE half and 16-byte aligned tables.
@@ -482,19 +516,27 @@ int launch_fused(const void* a, const void* b, int64_t m, int64_t n, int64_t k, 
   auto* A = static_cast<const uint8_t*>(a);
   auto* B = static_cast<const uint8_t*>(b);
   const int fast = fast_rope(p);
-  if (aligned) {
-    // The GEMM library's schedule for this output shape; 256 x 224 tiles do not hold whole
-    // heads, so the narrow schedule is not offered here.
-    int64_t full = -1;
-    if (gemm::detail::plan_schedule(false, false, m, n, device_cus(), full) == gemm::detail::SCHED_MIXED) {
-      const int64_t wgs = full + 2 * (tiles - full);
-      qk_mixed_kernel<MODE><<<dim3(static_cast<unsigned>(wgs)), block, 0, st>>>(A, B, (int)m, (int)n, kb,
-                                                                               static_cast<int>(full), sa, sb, p, fast);
-    } else {
-      qk_fused_kernel<MODE, true><<<grid, block, 0, st>>>(A, B, (int)m, (int)n, kb, sa, sb, p, fast);
-    }
+  // The plain GEMM's choice for this product.  Where it runs on ring tiles, so does this kernel, whose
+  // float sums then have the plain GEMM's bits.
+  const int tile = gemm::detail::plan_tile(MODE, m, n, kb, device_cus(), aligned).tile;
+  if (!aligned || tile == gemm::plan::TILE_128 || tile == gemm::plan::TILE_64 || tile == gemm::plan::TILE_64_DEEP) {
+    using R = gemm::detail::RingTiles<MODE>;
+    const dim3 wgs(static_cast<unsigned>(((m + 127) / 128) * (n / HEAD)));
+    if (aligned)
+      launch_kernel(qk_ring_kernel<typename R::T128, true>, wgs, dim3(512), st, A, B, (int)m, (int)n, kb, sa, sb, p, fast);
+    else
+      launch_kernel(qk_ring_kernel<typename R::U128, false>, wgs, dim3(512), st, A, B, (int)m, (int)n, kb, sa, sb, p, fast);
+    return launch_status("m5k_projection_qk_rope");
+  }
+  // The GEMM library's 256-row schedule for this output shape; 256 x 224 tiles do not hold whole
+  // heads, so the narrow schedule is not offered here.
+  int64_t full = -1;
+  if (gemm::detail::plan_schedule(false, false, m, n, device_cus(), full) == gemm::detail::SCHED_MIXED) {
+    const int64_t wgs = full + 2 * (tiles - full);
+    qk_mixed_kernel<MODE><<<dim3(static_cast<unsigned>(wgs)), block, 0, st>>>(A, B, (int)m, (int)n, kb,
+                                                                             static_cast<int>(full), sa, sb, p, fast);
   } else {
-    qk_fused_kernel<MODE, false><<<grid, block, 0, st>>>(A, B, (int)m, (int)n, kb, sa, sb, p, fast);
+    qk_fused_kernel<MODE><<<grid, block, 0, st>>>(A, B, (int)m, (int)n, kb, sa, sb, p, fast);
   }
   return launch_status("m5k_projection_qk_rope");
 }
@@ -547,6 +589,29 @@ extern "C" int m5k_qk_norm_rope(const void* projected, int64_t m, int64_t n, con
              rope_half, epsilon, static_cast<uint16_t*>(y), 0, nullptr, nullptr, nullptr};
   const int64_t groups = m * (n / HEAD);
   const int64_t blocks = (groups + 15) / 16;
+  M5K_REQUIRE(blocks <= 0x7FFFFFFF, "%s: input too large", name);
+  qk_norm_rope_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream)>>>(
+      static_cast<const uint16_t*>(projected), m, n, p, fast_rope(p));
+  return launch_status(name);
+}
+
+extern "C" int m5k_qkv_norm_rope(const void* projected, int64_t m, int64_t heads, const void* q_gamma,
+                                 const void* k_gamma, const void* cos, const void* sin, int rope_half, float epsilon,
+                                 void* q_out, void* k_out, void* v_out, void* stream) {
+  clear_error();
+  const char* name = "m5k_qkv_norm_rope";
+  M5K_REQUIRE(heads > 0 && heads <= 0x7FFFFFFF / (3 * HEAD), "%s: bad head count %lld", name, (long long)heads);
+  const int64_t n = heads * 3 * HEAD;
+  if (int rc = check_norm_args(m, n, q_gamma, cos, sin, rope_half, epsilon, q_out, name)) return rc;
+  M5K_REQUIRE(projected && aligned16(projected), "%s: projection must be a 16-byte aligned pointer", name);
+  M5K_REQUIRE(k_gamma && k_out && v_out, "%s: null pointer", name);
+  M5K_REQUIRE(aligned16(k_out) && aligned16(v_out), "%s: outputs must be 16-byte aligned", name);
+  QkParams p{static_cast<const uint16_t*>(q_gamma), static_cast<const uint16_t*>(cos),
+             static_cast<const uint16_t*>(sin),     rope_half,
+             epsilon,                               static_cast<uint16_t*>(q_out),
+             1,                                     static_cast<const uint16_t*>(k_gamma),
+             static_cast<uint16_t*>(k_out),         static_cast<uint16_t*>(v_out)};
+  const int64_t blocks = (m * (n / HEAD) + 15) / 16;
   M5K_REQUIRE(blocks <= 0x7FFFFFFF, "%s: input too large", name);
   qk_norm_rope_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, as_stream(stream)>>>(
       static_cast<const uint16_t*>(projected), m, n, p, fast_rope(p));

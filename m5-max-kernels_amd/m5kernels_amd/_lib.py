@@ -52,6 +52,7 @@ SIGNATURES = {
     "m5k_gemm_i8": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p, _p, _p, _p, _p, _p],
     "m5k_gemm_i8_acc": [_p, _p, _i64, _i64, _i64, _p, _p],
     "m5k_gemm_launch_plan": [_i32, _i64, _i64, _i32, _p, _p],
+    "m5k_gemm_tile_plan": [_i32, _i64, _i64, _i64, _i32, _i32, _p],
     "m5k_gemm_set_schedule": [_i32, _p],
     "m5k_gemm_i8_splitk": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p, _p, _p, _p, _p, _i32, _p, _i64, _p],
     "m5k_gemm_i8_splitk_noalloc": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p, _p, _p, _p, _p, _i32, _p],
@@ -67,6 +68,7 @@ SIGNATURES = {
     "m5k_gated_residual_add": [_p, _i32, _i64, _i64, _p, _i32, _p, _i32, _p, _p, _p],
     "m5k_projection_qk_rope": [_p, _p, _i32, _i64, _i64, _i64, _p, _p, _p, _p, _p, _i32, _f32, _p, _p],
     "m5k_qk_norm_rope": [_p, _i64, _i64, _p, _p, _p, _i32, _f32, _p, _p],
+    "m5k_qkv_norm_rope": [_p, _i64, _i64, _p, _p, _p, _p, _i32, _f32, _p, _p, _p, _p],
 }
 
 _LIB = None

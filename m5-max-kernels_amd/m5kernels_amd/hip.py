@@ -93,10 +93,12 @@ def _check_vector(t, n, dtype, message):
 
 
 def splitk_plan(m, n, k, cus=256, skinny=True):
-    """Number of K ranges per output tile for the W8A8 linear (1 = one workgroup per tile).
+    """Largest number of K ranges per output tile for the W8A8 linear (1 = one workgroup per tile): the
+    workspace that gemm() hands to the split entry points, which take as many ranges as pay on the tile
+    that they choose (csrc/gemm_plan.h).  It is sized for 256-row tiles:
 
     Shapes with few 256 x 256 tiles (short M) leave most of the 256 CUs idle; splitting K
-    aims at ~224 workgroups, each over at least 4 slabs of 64 bytes.  The INT32 partial
+    aims at one workgroup per CU, each over at least 4 slabs of 64 bytes.  The INT32 partial
     tiles cost 8 * splits * M * N bytes of extra traffic against the N * K bytes of weights,
     so splits also stay below K / (2 M).  (Measured on MI355X over M 16..512 and H3 widths:
     within ~10% of the best split count, 1.4-3.7x faster than one workgroup per tile.)
@@ -128,7 +130,7 @@ def splitk_plan(m, n, k, cus=256, skinny=True):
         if splits >= 2:
             return splits
     tiles = tiles_m * -(-n // 256)
-    splits = min(224 // tiles, slabs // 4, max(2, k // (2 * m)), 64)
+    splits = min(cus // tiles, slabs // 4, max(2, k // (2 * m)), 64)
     return splits if splits >= 2 else 1
 
 
@@ -176,8 +178,9 @@ _SCHEDULE_CODES = {name: i for i, name in enumerate(SCHEDULES)}
 def launch_override(schedule=None, splits=None):
     """Fix the gfx950 GEMM launch for the calls this thread makes inside the block: `schedule`
     ("plain", "mixed", "narrow" or "quad"; set in the library for this host thread with
-    m5k_gemm_set_schedule) and, for the W8A8 linear, the split-K count `splits` (1: no split;
-    the INT32 partials are exact, so every choice gives the same bits).  A forced schedule with
+    m5k_gemm_set_schedule) and, for the W8A8 linear, the largest split-K count `splits` (1: no split;
+    the library may take fewer K ranges; the INT32 partials are exact, so every choice gives the same
+    bits).  A forced schedule with
     `splits` None runs unsplit: the launch timed is the one named.  None keeps the library's own
     plan.  These are the knobs the harness tuner searches; both settings are thread-local."""
     if schedule is not None and schedule not in SCHEDULES:
@@ -217,6 +220,34 @@ def _cu_count(device):
     return _cu_count_of(device.index if device.index is not None else torch.cuda.current_device())
 
 
+TILES = ("256", "128", "64", "64-deep", "decode")
+
+
+@functools.lru_cache(maxsize=4096)
+def _tile_plan(mode, m, n, k, cus, aligned, forced):
+    """The library's tile for an [m, n, k] product (m5k_gemm_tile_plan; host only), cached per shape
+    and schedule settings `forced`, which the library reads itself."""
+    tile = ctypes.c_int(0)
+    lib = _lib.load()
+    if lib.m5k_gemm_tile_plan(_PLAN_DTYPES[mode], m, n, k, cus, int(aligned), ctypes.byref(tile)):
+        raise RuntimeError(lib.m5k_last_error().decode(errors="replace"))
+    return TILES[tile.value]
+
+
+def _environ_schedule():
+    environ = os.environ
+    return (environ.get("M5K_GEMM_MIXED_TILES"), environ.get("M5K_GEMM_NARROW_TILES"), environ.get("M5K_GEMM_SCHEDULE"))
+
+
+def tile_plan(mode, a, b):
+    """The tile that gemm(a, b, mode) runs without partial sums, by name (TILES)."""
+    m, k = a.shape
+    row = k * a.element_size()
+    aligned = row % 16 == 0 and row <= 1 << 23 and a.data_ptr() % 16 == 0 and b.data_ptr() % 16 == 0
+    return _tile_plan(mode, m, b.shape[0], k, _cu_count(a.device), aligned,
+                      (getattr(_override, "schedule", None), _environ_schedule()))
+
+
 @functools.lru_cache(maxsize=4096)
 def _i8_schedule(m, n, k, cus, env):
     """Host schedule of an aligned W8A8 linear, cached per shape, CU count and the library's
@@ -226,6 +257,8 @@ def _i8_schedule(m, n, k, cus, env):
     if env[2]:
         return 1, None  # a schedule forced from the environment runs unsplit, as named
     splits = splitk_plan(m, n, k, cus)
+    if splits > 1 and _tile_plan("int8", m, n, k, cus, True, (None, env)) == "decode":
+        splits = 1  # a few rows: the decode tile splits K inside its workgroups
     # The library's mixed and narrow launches refill a partial last round without INT32
     # partials and measured faster wherever both apply; the split-K tail takes the rest.
     tail = None
@@ -365,10 +398,7 @@ def gemm(
         elif aligned and getattr(_override, "schedule", None) is not None:
             splits = 1  # a forced schedule runs unsplit, without the tail split
         elif aligned:
-            environ = os.environ
-            env = (environ.get("M5K_GEMM_MIXED_TILES"), environ.get("M5K_GEMM_NARROW_TILES"),
-                   environ.get("M5K_GEMM_SCHEDULE"))
-            splits, tail = _i8_schedule(m, n, k, _cu_count(a.device), env)
+            splits, tail = _i8_schedule(m, n, k, _cu_count(a.device), _environ_schedule())
         if tail is not None:
             # Whole tile rows in full rounds, then the remaining rows split along K.  Every
             # row-indexed operand is sliced at the same row; both launches are bit-exact.

@@ -17,9 +17,20 @@ import struct
 import torch
 
 from . import _lib
-from .hip import gemm, splitk_plan
+from .hip import gemm, splitk_plan, tile_plan
 
 HEAD_DIM = 128
+
+
+def _staged(a, b, mode):
+    """Whether the projection runs as the plain GEMM and the staged postprocess: where the GEMM's best
+    tile is smaller than a head (few rows: 128 x 7168 x 5376 INT8 14 us + 4 us against 26 us fused on
+    one-head tiles), or a split over K.  The fused kernel's tiles otherwise: it takes the plain GEMM's
+    choice between one-head and 256-row tiles.  Both give the same bits."""
+    tile = tile_plan(mode, a, b)
+    if tile == "256":
+        return mode == "int8" and splitk_plan(a.shape[0], b.shape[0], a.shape[1]) > 1
+    return tile != "128"
 
 
 def _epsilon(epsilon):
@@ -106,14 +117,12 @@ def projection_qk_rope(
         raise ValueError("BF16 projection does not accept quantization scales")
     rope_half, eps32 = _validate_norm(m, n, gamma, cos, sin, epsilon)
     _validate_tile(tile)
-    if mode == "int8" and splitk_plan(m, n, k) > 1:
-        # Few output tiles (short M): the split-K W8A8 projection to BF16, then the staged
-        # postprocess.  Both are the fused kernel's arithmetic, so the bits are the same.
-        projected = gemm(a, b, "int8", a_scales=a_scales, b_scales=b_scales, output_dtype=torch.bfloat16)
-        return qk_norm_rope(projected, gamma, cos, sin, epsilon=epsilon)
-    epsilon = eps32
     a = _lib.device_tensor(a, "a")
     b = _lib.device_tensor(b, "b")
+    if _staged(a, b, mode):
+        projected = gemm(a, b, mode, a_scales=a_scales, b_scales=b_scales, output_dtype=torch.bfloat16)
+        return qk_norm_rope(projected, gamma, cos, sin, epsilon=epsilon)
+    epsilon = eps32
     gamma, cos, sin = _tables(gamma, cos, sin)
     y = torch.empty((n // HEAD_DIM, m, HEAD_DIM), dtype=torch.bfloat16, device=a.device)
     if mode == "int8":
@@ -184,7 +193,17 @@ def projection_qkv_rope(a, w, q_gamma, k_gamma, cos, sin, mode="int8", *, a_scal
     w = _lib.device_tensor(w, "w")
     q_gamma, cos, sin = _tables(q_gamma, cos, sin)
     k_gamma = _lib.aligned_device_tensor(k_gamma, "k_gamma")
+    staged = _staged(a, w, mode)
+    if staged:
+        projected = gemm(a, w, mode, a_scales=a_scales, b_scales=w_scales, output_dtype=torch.bfloat16)
     q, kk, v = (torch.empty((heads, m, HEAD_DIM), dtype=torch.bfloat16, device=a.device) for _ in range(3))
+    if staged:
+        _lib.call(
+            "m5k_qkv_norm_rope",
+            _lib.ptr(projected), m, heads, _lib.ptr(q_gamma), _lib.ptr(k_gamma), _lib.ptr(cos), _lib.ptr(sin),
+            int(rope_half), float(epsilon), _lib.ptr(q), _lib.ptr(kk), _lib.ptr(v), _lib.stream_of(a),
+        )
+        return q, kk, v
     if mode == "int8":
         a_scales = _lib.device_tensor(a_scales, "a_scales")
         w_scales = _lib.device_tensor(w_scales, "w_scales")

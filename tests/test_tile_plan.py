@@ -1,0 +1,51 @@
+"""The GEMM's tile choice (m5k_gemm_tile_plan; host only)."""
+
+import ctypes
+import random
+
+import pytest
+
+from m5kernels_amd import _lib, hip
+
+
+def _plan(mode, m, n, k, aligned=True):
+    return hip._tile_plan.__wrapped__(mode, m, n, k, 256, aligned, None)
+
+
+def test_tile_by_shape():
+    for mode in ("int8", "fp8"):
+        assert _plan(mode, 1, 4096, 4096) == "decode"
+        assert _plan(mode, 128, 4096, 4096) == "64-deep"
+        assert _plan(mode, 256, 7168, 5376) == "64"
+        assert _plan(mode, 512, 7168, 5376) == "128"
+        assert _plan(mode, 4096, 4096, 16384) == "256"
+    assert _plan("bf16", 128, 5376, 5120) == "64-deep"
+    assert _plan("fp32", 128, 5376, 5120) == "256"
+
+
+def test_rules_over_random_shapes():
+    rng = random.Random(5)
+    for _ in range(2000):
+        m, n, k = (round(10 ** rng.uniform(0, 4.2)) for _ in range(3))
+        for mode, size in (("int8", 1), ("fp8", 1), ("bf16", 2), ("fp16", 2)):
+            tile = _plan(mode, m, n, k)
+            assert tile != "decode" or m <= 32
+            if mode != "int8" and k * size < 1024:
+                assert tile == "256"  # one FP32 chain over K
+            loose = _plan(mode, m, n, k, aligned=False)
+            assert loose == "256" if mode == "fp8" else loose in ("64", "128")
+        assert _plan("bf16", m, n, k) == _plan("fp16", m, n, k)
+
+
+def test_a_forced_schedule_keeps_the_256_row_tiles():
+    with hip.launch_override("plain"):
+        assert _plan("int8", 1, 4096, 4096) == "256"
+    assert _plan("int8", 1, 4096, 4096) == "decode"
+
+
+def test_argument_checks():
+    lib, tile = _lib.load(), ctypes.c_int(0)
+    assert lib.m5k_gemm_tile_plan(_lib.I8, 0, 4, 4, 256, 1, ctypes.byref(tile)) == 1
+    assert lib.m5k_gemm_tile_plan(_lib.I8, 4, 4, 4, 0, 1, ctypes.byref(tile)) == 1
+    assert lib.m5k_gemm_tile_plan(_lib.I32, 4, 4, 4, 256, 1, ctypes.byref(tile)) == 1
+    assert lib.m5k_gemm_tile_plan(_lib.I8, 4, 4, 4, 256, 1, None) == 1
