@@ -37,7 +37,7 @@ struct Choice {
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 inline double split_us(int64_t m, int64_t n, int splits) {
-  return splits > 1 ? 3.0 + 8.0 * splits * static_cast<double>(m) * static_cast<double>(n) / 6.0e6 : 0.0;
+  return splits > 1 ? 5.0 + 8.0 * splits * static_cast<double>(m) * static_cast<double>(n) / 6.0e6 : 0.0;
 }
 
 // max(a tile's own time, the weight's stream), the former breaking ties.
