@@ -9,8 +9,10 @@
 //   code  = peak == 0 ? 0 : clamp(rint((z / peak) * 127), -127, 127)
 // There is no additive shift and no reduced-precision intermediate, so the positive inverse
 // RMS moves only the scales (fold = true) and the row peak and statistics can share one
-// barrier.  One workgroup of 4 wave64 per row; for B >= 32 a lane holds NCH chunks of EPC
-// consecutive elements in VGPRs, for B = 1 (any K) the row is read through the cache per pass.
+// barrier.  One workgroup of 4 wave64 per row; a lane holds NCH chunks of EPC consecutive elements in
+// VGPRs.  B = 1 takes the same kernel without the butterflies where its chunks of 8 apply (K % 8 == 0,
+// aligned operands, K <= 16384); any other K, and operands without that alignment, read the row through
+// the cache element by element, once per pass ([512, 5376] BF16: 14.3 us, against 5.2 us in registers).
 #include "hadamard_core.h"
 
 namespace m5k {
@@ -72,12 +74,25 @@ __device__ __forceinline__ float2 block_max_sum(float m, float s, float2* lds) {
   return r;
 }
 
-// Block-Hadamard variant (B >= 32, K % B == 0).
+// Elements per chunk and the transform's final factor; B = 1: no transform.
+template <int B>
+__device__ __host__ constexpr int chunk_elems() {
+  if constexpr (B == 1) return 8;
+  else return Shape<B>::EPC;
+}
+
+template <int B>
+__device__ constexpr float transform_factor() {
+  if constexpr (B == 1) return 1.0f;
+  else return hadamard::inv_sqrt_block<B>();
+}
+
+// Register-resident rows (B >= 32: K % B == 0; B = 1: K % 8 == 0).
 template <int XDT, int B, int NCH, bool FOLD>
 __global__ __launch_bounds__(kThreads) void rms_quant_block_kernel(RmsParams p) {
   __shared__ float red[2 * kWaves];  // unfolded: statistics, then peak
   __shared__ float2 red2[kWaves];    // folded: peak and sum of squares
-  constexpr int EPC = Shape<B>::EPC;
+  constexpr int EPC = chunk_elems<B>();
   constexpr int NV = NCH * EPC;
   const int64_t row = blockIdx.x;
   const int tid = threadIdx.x;
@@ -144,7 +159,7 @@ __global__ __launch_bounds__(kThreads) void rms_quant_block_kernel(RmsParams p) 
         z[8 * h + r] = FOLD ? (x * gr) * s : ((x * inv) * gr) * s;
       }
     }
-    hadamard::butterflies<B, false>(z);
+    if constexpr (B > 1) hadamard::butterflies<B, false>(z);
 #pragma unroll
     for (int r = 0; r < EPC; r += 2) {
       v[i * EPC + r] = z[r];
@@ -157,7 +172,7 @@ __global__ __launch_bounds__(kThreads) void rms_quant_block_kernel(RmsParams p) 
   // rint(fl(fl(z / peak) * 127)), three roundings of z' * m for m = 127 c / peak, bracketed
   // by the estimate m~ = fl(c * fl(127 / peak)) (two roundings; 0 for a zero or infinite peak,
   // where every finite z codes to 0).
-  constexpr float c = hadamard::inv_sqrt_block<B>();
+  constexpr float c = transform_factor<B>();
   if constexpr (FOLD) {
     // Peak and sum of squares share one barrier; only the lane that writes the scale needs
     // the inverse RMS.
@@ -187,7 +202,7 @@ __global__ __launch_bounds__(kThreads) void rms_quant_block_kernel(RmsParams p) 
   }
 }
 
-// B = 1 (no transform, any K): three passes over the cached row.
+// B = 1 for any K and alignment: three passes over the cached row.
 template <int XDT, bool FOLD>
 __global__ __launch_bounds__(kThreads) void rms_quant_plain_kernel(RmsParams p) {
   __shared__ float red[3 * kWaves];
@@ -221,7 +236,7 @@ __global__ __launch_bounds__(kThreads) void rms_quant_plain_kernel(RmsParams p) 
 
 template <int XDT, int B, bool FOLD>
 int launch_block(const RmsParams& p, int64_t rows, hipStream_t st) {
-  const int64_t per_thread = (p.k / Shape<B>::EPC + kThreads - 1) / kThreads;
+  const int64_t per_thread = (p.k / chunk_elems<B>() + kThreads - 1) / kThreads;
   const dim3 grid(static_cast<unsigned>(rows)), block(kThreads);
   if (per_thread <= 1) rms_quant_block_kernel<XDT, B, 1, FOLD><<<grid, block, 0, st>>>(p);
   else if (per_thread <= 2) rms_quant_block_kernel<XDT, B, 2, FOLD><<<grid, block, 0, st>>>(p);
@@ -230,7 +245,7 @@ int launch_block(const RmsParams& p, int64_t rows, hipStream_t st) {
   else if (per_thread <= 8) rms_quant_block_kernel<XDT, B, 8, FOLD><<<grid, block, 0, st>>>(p);
   else {
     set_error("m5k_rms_quantize: K=%lld exceeds the register-resident row limit %d", (long long)p.k,
-              8 * kThreads * Shape<B>::EPC);
+              8 * kThreads * chunk_elems<B>());
     return M5K_EINVAL;
   }
   return launch_status("m5k_rms_quantize");
@@ -239,8 +254,12 @@ int launch_block(const RmsParams& p, int64_t rows, hipStream_t st) {
 template <int XDT, bool FOLD>
 int by_block(int block, const RmsParams& p, int64_t rows, hipStream_t st) {
   switch (block) {
-    case 1: rms_quant_plain_kernel<XDT, FOLD><<<dim3(static_cast<unsigned>(rows)), dim3(kThreads), 0, st>>>(p);
-            return launch_status("m5k_rms_quantize");
+    case 1:
+      if (p.k % 8 == 0 && p.k <= 8 * kThreads * 8 && aligned16(p.x) && aligned16(p.gamma) &&
+          (reinterpret_cast<uintptr_t>(p.signs) & 7u) == 0 && (reinterpret_cast<uintptr_t>(p.q) & 7u) == 0)
+        return launch_block<XDT, 1, FOLD>(p, rows, st);
+      rms_quant_plain_kernel<XDT, FOLD><<<dim3(static_cast<unsigned>(rows)), dim3(kThreads), 0, st>>>(p);
+      return launch_status("m5k_rms_quantize");
     case 32: return launch_block<XDT, 32, FOLD>(p, rows, st);
     case 64: return launch_block<XDT, 64, FOLD>(p, rows, st);
     case 128: return launch_block<XDT, 128, FOLD>(p, rows, st);
