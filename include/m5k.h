@@ -103,6 +103,10 @@ int m5k_quantize_mxint8(const void* x, int x_dtype, int64_t rows, int64_t k, int
 int m5k_mxint8_to_bf16(const int8_t* q, const uint8_t* exponents, int64_t rows, int64_t k, void* y,
                        void* stream);
 
+/* The same for both operands of a product, codes a [m,k] and b [n,k], in one launch. */
+int m5k_mxint8_pair_to_bf16(const int8_t* qa, const uint8_t* ea, int64_t m, const int8_t* qb, const uint8_t* eb,
+                            int64_t n, int64_t k, void* ya, void* yb, void* stream);
+
 /*
  * W8A8 linear.  Replaces metal.gemm(a, b, "int8", ...) (src/m5kernels/metal.py:158-269,
  * epilogues :88-128).  a: [m,k] int8, b: [n,k] int8 (weights, K-contiguous).

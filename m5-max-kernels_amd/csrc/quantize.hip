@@ -227,14 +227,26 @@ __global__ __launch_bounds__(kThreads) void quantize_mx_kernel(const uint8_t* __
 }
 
 // MXINT8 codes to BF16 values code * 2^(e - 127): exact (|code| <= 127 fits the BF16
-// significand), 8 elements per thread.
-__global__ __launch_bounds__(kThreads) void mx_to_bf16_kernel(const int8_t* __restrict__ q,
-                                                              const uint8_t* __restrict__ s, int64_t groups,
-                                                              uint16_t* __restrict__ y) {
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  if (t >= groups) return;
-  const uint2 w = *reinterpret_cast<const uint2*>(q + t * 8);
-  const int e = static_cast<int>(s[t >> 2]) - 127;
+// significand), 8 elements per thread.  Two matrices, the GEMM's operands, in one launch: the smaller
+// one's threads run beside the larger one's instead of in a launch of their own ([1024, 4096] and
+// [4096, 4096]: 12.0 us against 4.7 + 9.0 us and the gap between them).
+struct MxMatrix {
+  const int8_t* q;
+  const uint8_t* s;
+  uint16_t* y;
+  int64_t groups;  // of 8 elements
+};
+
+__global__ __launch_bounds__(kThreads) void mx_to_bf16_kernel(MxMatrix first, MxMatrix second) {
+  int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
+  MxMatrix a = first;
+  if (t >= first.groups) {
+    t -= first.groups;
+    a = second;
+    if (t >= second.groups) return;
+  }
+  const uint2 w = *reinterpret_cast<const uint2*>(a.q + t * 8);
+  const int e = static_cast<int>(a.s[t >> 2]) - 127;
   uint32_t out[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -244,7 +256,14 @@ __global__ __launch_bounds__(kThreads) void mx_to_bf16_kernel(const int8_t* __re
     const float hi = ldexpf(static_cast<float>(static_cast<int8_t>((word >> (sh + 8)) & 0xFFu)), e);
     out[i] = f32x2_to_bf16x2(lo, hi);
   }
-  *reinterpret_cast<uint4*>(y + t * 8) = make_uint4(out[0], out[1], out[2], out[3]);
+  *reinterpret_cast<uint4*>(a.y + t * 8) = make_uint4(out[0], out[1], out[2], out[3]);
+}
+
+int launch_mx_to_bf16(const MxMatrix& first, const MxMatrix& second, hipStream_t st, const char* name) {
+  const int64_t blocks = (first.groups + second.groups + kThreads - 1) / kThreads;
+  M5K_REQUIRE(blocks <= 0x7FFFFFFF, "%s: input too large", name);
+  mx_to_bf16_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, st>>>(first, second);
+  return launch_status(name);
 }
 
 template <int DT, int MODE, int KT, int CPT>
@@ -340,10 +359,21 @@ extern "C" int m5k_mxint8_to_bf16(const int8_t* q, const uint8_t* exponents, int
   M5K_REQUIRE(rows > 0 && k > 0 && k % 32 == 0, "%s: shape [%lld,%lld] needs K a positive multiple of 32", name,
               (long long)rows, (long long)k);
   M5K_REQUIRE((reinterpret_cast<uintptr_t>(q) & 7u) == 0 && aligned16(y), "%s: misaligned buffers", name);
-  const int64_t groups = rows * k / 8;
-  const int64_t blocks = (groups + kThreads - 1) / kThreads;
-  M5K_REQUIRE(blocks <= 0x7FFFFFFF, "%s: input too large", name);
-  mx_to_bf16_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, as_stream(stream)>>>(
-      q, exponents, groups, static_cast<uint16_t*>(y));
-  return launch_status(name);
+  return launch_mx_to_bf16(MxMatrix{q, exponents, static_cast<uint16_t*>(y), rows * k / 8},
+                           MxMatrix{nullptr, nullptr, nullptr, 0}, as_stream(stream), name);
+}
+
+extern "C" int m5k_mxint8_pair_to_bf16(const int8_t* qa, const uint8_t* ea, int64_t m, const int8_t* qb,
+                                       const uint8_t* eb, int64_t n, int64_t k, void* ya, void* yb, void* stream) {
+  using namespace m5k;
+  clear_error();
+  const char* name = "m5k_mxint8_pair_to_bf16";
+  M5K_REQUIRE(qa && ea && qb && eb && ya && yb, "%s: null pointer", name);
+  M5K_REQUIRE(m > 0 && n > 0 && k > 0 && k % 32 == 0, "%s: shape m=%lld n=%lld k=%lld needs K a positive multiple of 32",
+              name, (long long)m, (long long)n, (long long)k);
+  M5K_REQUIRE((reinterpret_cast<uintptr_t>(qa) & 7u) == 0 && (reinterpret_cast<uintptr_t>(qb) & 7u) == 0 &&
+                  aligned16(ya) && aligned16(yb),
+              "%s: misaligned buffers", name);
+  return launch_mx_to_bf16(MxMatrix{qa, ea, static_cast<uint16_t*>(ya), m * k / 8},
+                           MxMatrix{qb, eb, static_cast<uint16_t*>(yb), n * k / 8}, as_stream(stream), name);
 }

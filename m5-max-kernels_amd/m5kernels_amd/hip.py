@@ -492,15 +492,11 @@ def gemm(
     return c
 
 
-def _mx_to_bf16(q, e, name):
+def _mx_operand(q, e, name):
     rows, k = q.shape
     if q.dtype != torch.int8 or e.dtype != torch.uint8 or tuple(e.shape) != (rows, k // 32):
         raise ValueError(f"MXINT8 {name} needs int8 codes [R,K] and uint8 exponents [R,K/32]")
-    q = _lib.device_tensor(q, name)
-    e = _lib.device_tensor(e, name + "_scales")
-    y = torch.empty((rows, k), dtype=torch.bfloat16, device=q.device)
-    _lib.call("m5k_mxint8_to_bf16", _lib.ptr(q), _lib.ptr(e), rows, k, _lib.ptr(y), _lib.stream_of(q))
-    return y
+    return _lib.device_tensor(q, name), _lib.device_tensor(e, name + "_scales")
 
 
 def _gemm_mxint8(a, b, a_scales, b_scales, output_dtype):
@@ -508,16 +504,22 @@ def _gemm_mxint8(a, b, a_scales, b_scales, output_dtype):
     2^(ea-127) 2^(eb-127) sum_k a b, FP32 accumulation.  Both operands expand exactly to BF16
     (|code| <= 127 times a power of two) and run on the BF16 MFMA GEMM."""
     m, k = a.shape
+    n = b.shape[0]
     if k % 32:
         raise ValueError("MXINT8 requires K divisible by 32")
     out_dtype = output_dtype or torch.float32
     if out_dtype not in _FLOAT_DTYPES:
         raise ValueError("output_dtype must be float16, bfloat16 or float32")
-    ab = _mx_to_bf16(a, a_scales, "a")
-    bb = _mx_to_bf16(b, b_scales, "b")
-    c = torch.empty((m, b.shape[0]), dtype=out_dtype, device=ab.device)
-    _lib.call("m5k_gemm_float", _lib.ptr(ab), _lib.ptr(bb), _lib.BF16, m, b.shape[0], k, _lib.ptr(c),
-              _lib.dtype_code(c), None, None, None, _lib.stream_of(ab))
+    a, a_scales = _mx_operand(a, a_scales, "a")
+    b, b_scales = _mx_operand(b, b_scales, "b")
+    ab = torch.empty((m, k), dtype=torch.bfloat16, device=a.device)
+    bb = torch.empty((n, k), dtype=torch.bfloat16, device=a.device)
+    stream = _lib.stream_of(a)
+    _lib.call("m5k_mxint8_pair_to_bf16", _lib.ptr(a), _lib.ptr(a_scales), m, _lib.ptr(b), _lib.ptr(b_scales), n, k,
+              _lib.ptr(ab), _lib.ptr(bb), stream)
+    c = torch.empty((m, n), dtype=out_dtype, device=a.device)
+    _lib.call("m5k_gemm_float", _lib.ptr(ab), _lib.ptr(bb), _lib.BF16, m, n, k, _lib.ptr(c),
+              _lib.dtype_code(c), None, None, None, stream)
     return c
 
 
