@@ -192,6 +192,13 @@ int m5k_gemm_launch_plan(int ab_dtype, int64_t m, int64_t n, int cus, int* sched
 int m5k_gemm_set_schedule(int schedule, int* previous);
 
 /*
+ * What decides the calling thread's schedules besides the shape, as one value (a key for host-side
+ * plan caches; no counterpart in the reference): bits 0-2 the thread's forced schedule + 1, bit 3 a
+ * schedule in M5K_GEMM_SCHEDULE, bits 4 and 5 M5K_GEMM_MIXED_TILES=0 and M5K_GEMM_NARROW_TILES=0.
+ */
+int m5k_gemm_schedule_state(void);
+
+/*
  * Tile of the MFMA GEMMs for an [m,n,k] product (host only, launches nothing; no counterpart in the
  * reference).  `aligned`: row bytes a multiple of 16 and at most 2^23, 16-byte aligned bases.  *tile
  * receives

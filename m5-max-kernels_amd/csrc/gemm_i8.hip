@@ -60,6 +60,16 @@ extern "C" int m5k_gemm_launch_plan(int ab_dtype, int64_t m, int64_t n, int cus,
   return M5K_OK;
 }
 
+extern "C" int m5k_gemm_schedule_state(void) {
+  auto off = [](const char* name) {
+    const char* env = std::getenv(name);
+    return env != nullptr && env[0] == '0';
+  };
+  const char* forced = std::getenv("M5K_GEMM_SCHEDULE");
+  return (g_thread_schedule + 1) | (forced != nullptr && forced[0] != '\0' ? 8 : 0) |
+         (off("M5K_GEMM_MIXED_TILES") ? 16 : 0) | (off("M5K_GEMM_NARROW_TILES") ? 32 : 0);
+}
+
 extern "C" int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int* tile) {
   clear_error();
   const char* name = "m5k_gemm_tile_plan";

@@ -9,13 +9,16 @@ from __future__ import annotations
 
 import ctypes
 import functools
+import importlib.util
 import re
+import warnings
 from numbers import Integral, Real
 from pathlib import Path
 
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent.parent / "lib" / "libm5k.so"
+FAST_PATH = LIB_PATH.with_name("m5k_fast.so")
 
 F32, F16, BF16, I8, U8, I32 = 0, 1, 2, 3, 4, 5
 QUANT_INT8, QUANT_FP8 = 0, 1
@@ -55,6 +58,7 @@ SIGNATURES = {
     "m5k_gemm_launch_plan": [_i32, _i64, _i64, _i32, _p, _p],
     "m5k_gemm_tile_plan": [_i32, _i64, _i64, _i64, _i32, _i32, _p],
     "m5k_gemm_set_schedule": [_i32, _p],
+    "m5k_gemm_schedule_state": [],
     "m5k_gemm_i8_splitk": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p, _p, _p, _p, _p, _i32, _p, _i64, _p],
     "m5k_gemm_i8_splitk_noalloc": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p, _p, _p, _p, _p, _i32, _p],
     "m5k_gemm_f8": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p],
@@ -98,6 +102,23 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
     if path is None:
         _LIB = lib
     return lib
+
+
+def load_fast():
+    """The native front of quantize() and gemm() (binding/fast_ops.cpp), linked against libm5k.so, or
+    None where the libraries have not been built.  One that does not load (left from an older build)
+    warns: the same kernels then run with the checks in Python, and this package still imports, so that
+    it can be built again."""
+    if not (FAST_PATH.exists() and LIB_PATH.exists()) or _current_raw_stream is None:
+        return None
+    spec = importlib.util.spec_from_file_location("m5k_fast", FAST_PATH)
+    try:
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+    except ImportError as e:
+        warnings.warn(f"{FAST_PATH.name} does not load ({e}); build the package again", RuntimeWarning)
+        return None
+    return module
 
 
 def call(name: str, *args) -> None:

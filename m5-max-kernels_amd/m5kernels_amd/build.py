@@ -2,7 +2,8 @@
 
 Every translation unit under ``csrc/`` is compiled to an object under ``_build/``
 (in parallel), then linked into ``lib/libm5k.so`` next to this package.  The measurement
-kernels under ``diag/`` (bench.py's MFMA ceiling) go into ``lib/libm5k_diag.so``.  Flags:
+kernels under ``diag/`` (bench.py's MFMA ceiling) go into ``lib/libm5k_diag.so``, the native front of quantize() and gemm() under ``binding/`` (host code, against
+torch's headers) into ``lib/m5k_fast.so``.  Flags:
 
 * ``--offload-arch=gfx950`` only: MI355X is the single target.
 * ``-ffp-contract=off``: no FMA contraction, so FP32 epilogues and normalization keep
@@ -18,6 +19,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -29,6 +31,8 @@ BUILD_DIR = REPO_ROOT / "_build" / "libm5k"
 LIB_PATH = PKG_ROOT / "lib" / "libm5k.so"
 DIAG_DIR = PKG_ROOT / "diag"
 DIAG_LIB_PATH = PKG_ROOT / "lib" / "libm5k_diag.so"
+FAST_SRC = PKG_ROOT / "binding" / "fast_ops.cpp"
+FAST_PATH = PKG_ROOT / "lib" / "m5k_fast.so"
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -77,18 +81,51 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     LIB_PATH.parent.mkdir(parents=True, exist_ok=True)
     srcs = sources()
     jobs = jobs or min(len(srcs), max(1, min(8, os.cpu_count() or 1)))
+    fast_obj = BUILD_DIR / "fast_ops.o"
     with ThreadPoolExecutor(max_workers=jobs) as pool:
+        fast = pool.submit(_compile_fast, fast_obj, force)
         objs = list(pool.map(lambda s: _compile(s, force), srcs))
+        fast.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link of libm5k.so failed:\n{proc.stderr[-4000:]}")
     os.replace(tmp, LIB_PATH)
+    _link_fast(fast_obj)
     build_diag()
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources, and {DIAG_LIB_PATH}", file=sys.stderr)
     return LIB_PATH
+
+
+def _compile_fast(obj: Path, force: bool) -> None:
+    """The native front of quantize() and gemm(): host code against torch's headers."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    newest_dep = max(p.stat().st_mtime for p in [FAST_SRC, *INCLUDE.glob("*.h")])
+    if not force and obj.exists() and obj.stat().st_mtime >= newest_dep:
+        return
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+           f"-I{sysconfig.get_paths()['include']}", *(f"-isystem{p}" for p in include_paths()),
+           "-c", str(FAST_SRC), "-o", str(obj)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"compile of {FAST_SRC.name} failed:\n{proc.stderr[-4000:]}")
+
+
+def _link_fast(obj: Path) -> None:
+    from torch.utils.cpp_extension import library_paths
+
+    tmp = FAST_PATH.with_suffix(".so.tmp")
+    cmd = ["g++", "-shared", "-o", str(tmp), str(obj), f"-L{LIB_PATH.parent}", "-lm5k", "-Wl,-rpath,$ORIGIN",
+           *(f"-L{p}" for p in library_paths()), "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"link of {FAST_PATH.name} failed:\n{proc.stderr[-4000:]}")
+    os.replace(tmp, FAST_PATH)
 
 
 def build_diag() -> Path:

@@ -50,6 +50,10 @@ def quantize(x, mode, tag="packed"):
     scale, returned as uint8 exponent bytes [rows, K/32] (e + 127, numerics.py:33-41).
     Mirrors metal.quantize (metal.py:27-44).
     """
+    if _fast is not None:
+        done = _fast.quantize(x, mode)
+        if done is not None:
+            return done
     rows, k = x.shape
     if mode == "mxint8":
         if k % 32:
@@ -267,6 +271,17 @@ def _i8_schedule(m, n, k, cus, env):
     return splits, tail
 
 
+def _native_splits(mode, m, n, k, index):
+    """K ranges of an aligned INT8 or FP8 product on device `index` for the native front, which keeps
+    them per shape and m5k_gemm_schedule_state; 0 where this module runs the product itself (a tail
+    split's two launches)."""
+    cus = _cu_count_of(index)
+    if mode == "fp8":
+        return _f8_splits(m, n, k, cus, os.environ.get("M5K_GEMM_SCHEDULE"))
+    splits, tail = _i8_schedule(m, n, k, cus, _environ_schedule())
+    return 0 if tail is not None else splits
+
+
 @functools.lru_cache(maxsize=4096)
 def _f8_splits(m, n, k, cus, forced):
     """K ranges per tile of an aligned FP8 linear (1: the plain launch), cached per shape, CU
@@ -274,11 +289,14 @@ def _f8_splits(m, n, k, cus, forced):
     return 1 if forced else splitk_plan(m, n, k, cus, skinny=False)
 
 
+_TILE = (64, 64, 4, 1)
+
+
 def gemm(
     a,
     b,
     mode="bf16",
-    tile=(64, 64, 4, 1),
+    tile=_TILE,
     a_scales=None,
     b_scales=None,
     output_dtype=None,
@@ -297,6 +315,10 @@ def gemm(
     [P,N] with gate_row_map[M]); that requires BF16 output and cannot be combined with
     a bias.  output_dtype defaults to float32.  Mirrors metal.gemm (metal.py:158-269).
     """
+    if _fast is not None and tile is _TILE and getattr(_override, "splits", None) is None:
+        c = _fast.gemm(a, b, mode, a_scales, b_scales, output_dtype, bias, bias_row_map, residual, gate, gate_row_map)
+        if c is not None:
+            return c
     m, k = a.shape
     n, kb = b.shape
     if k != kb:
@@ -538,3 +560,8 @@ def gemm_i8_accumulators(a, b):
     acc = torch.empty((m, n), dtype=torch.int32, device=a.device)
     _lib.call("m5k_gemm_i8_acc", _lib.ptr(a), _lib.ptr(b), m, n, k, _lib.ptr(acc), _lib.stream_of(a))
     return acc
+
+
+_fast = _lib.load_fast()
+if _fast is not None:
+    _fast.bind(_lib._current_raw_stream, _native_splits)
