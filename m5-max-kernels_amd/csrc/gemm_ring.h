@@ -235,30 +235,40 @@ __device__ __forceinline__ void mainloop(const uint8_t* __restrict__ A, const ui
   stage_barrier();
 }
 
-// One 16-byte chunk at any byte address; `left` bytes of it lie before the row's end (the rest
-// reads as zero, and no byte at or past the row's end is touched).
-__device__ __forceinline__ v4i load_chunk(const uint8_t* p, int64_t left) {
+// The 16 bytes at any byte address p of a row of which `left` bytes remain there; bytes past the row's
+// end read as zero, and none of them is touched: a partial chunk is loaded so that it ends with the
+// row, and shifted down (rows of under 16 bytes: byte by byte).
+__device__ __forceinline__ v4i load_tail_chunk(const uint8_t* p, int64_t left, int64_t kb) {
   v4i v = {0, 0, 0, 0};
-  if (left >= 16) {
-    __builtin_memcpy(&v, p, 16);
-  } else if (left > 0) {
+  if (left <= 0) return v;
+  if (kb < 16) {
     uint32_t w[4] = {0, 0, 0, 0};
 #pragma unroll
     for (int e = 0; e < 15; ++e)
       if (e < left) w[e >> 2] |= static_cast<uint32_t>(p[e]) << (8 * (e & 3));
-    v = v4i{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])};
+    return v4i{static_cast<int>(w[0]), static_cast<int>(w[1]), static_cast<int>(w[2]), static_cast<int>(w[3])};
   }
+  const int drop = left >= 16 ? 0 : static_cast<int>(16 - left);  // bytes of the load before p
+  uint64_t q[2];
+  __builtin_memcpy(q, p - drop, 16);
+  const int s = 8 * (drop & 7);
+  const uint64_t lo = drop >= 8 ? q[1] : q[0], hi = drop >= 8 ? 0 : q[1];
+  q[0] = (lo >> s) | (s ? hi << (64 - s) : 0);
+  q[1] = hi >> s;
+  __builtin_memcpy(&v, q, 16);
   return v;
 }
 
 // The same tile for rows or bases that are not 16-byte aligned (odd K): a wave loads its share of a
-// stage into registers with unaligned 16-byte loads, one stage ahead of the LDS writes, into the
-// layout that mainloop's loads give.  Two stage buffers.  (Byte by byte through one buffer, with a
-// full wait per stage, a 300 x 520 x 1000 INT8 product took 127 us.)
+// stage into registers with unaligned 16-byte loads, AHEAD stages before they are written to the LDS,
+// in the layout that mainloop's loads give.  Two stage buffers.  300 x 520 x 1000 INT8: 127 us byte by
+// byte through one buffer with a full wait per stage, 9.2 us one stage ahead with a byte-by-byte tail,
+// 8.3 us this way (aligned operands of that size: 5.5 us).
 template <class C>
 __device__ __forceinline__ void mainloop_unaligned(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M,
                                                    int N, int64_t Kb, int m0, int n0, Acc<C>& acc, uint8_t* lds) {
   static_assert(C::NST >= 2 && C::PLANES == 1, "two buffers of one 128-byte plane");
+  constexpr int AHEAD = 3;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const WaveId id(wave);
@@ -275,40 +285,55 @@ __device__ __forceinline__ void mainloop_unaligned(const uint8_t* __restrict__ A
     lchunk[i] = ((lane & 7) ^ swz(r)) << 4;
     src[i] = (is_b ? B : A) + (in[i] ? row : 0) * Kb + lchunk[i];
   }
-  v4i regs[C::Q];
-  auto load = [&](int64_t kt) {
+  const int64_t count = stages<C>(Kb), whole = Kb / BKB;
+  v4i regs[AHEAD][C::Q];
+  auto load = [&](v4i (&r)[C::Q], int64_t kt) {
 #pragma unroll
-    for (int i = 0; i < C::Q; ++i)
-      regs[i] = load_chunk(src[i] + kt * BKB, in[i] ? Kb - kt * BKB - lchunk[i] : 0);
+    for (int i = 0; i < C::Q; ++i) {
+      r[i] = v4i{0, 0, 0, 0};
+      if (kt < whole) {  // uniform
+        if (in[i]) __builtin_memcpy(&r[i], src[i] + kt * BKB, 16);
+      } else if (kt < count) {
+        r[i] = load_tail_chunk(src[i] + kt * BKB, in[i] ? Kb - kt * BKB - lchunk[i] : 0, Kb);
+      }
+    }
   };
-  auto store = [&](int buf) {
+  auto store = [&](const v4i (&r)[C::Q], int buf) {
 #pragma unroll
     for (int i = 0; i < C::Q; ++i)
-      *reinterpret_cast<v4i*>(lds + buf * C::STAGE + (wave * C::Q + i) * 1024 + lane * 16) = regs[i];
+      *reinterpret_cast<v4i*>(lds + buf * C::STAGE + (wave * C::Q + i) * 1024 + lane * 16) = r[i];
   };
 #pragma unroll
   for (int i = 0; i < C::FM; ++i)
 #pragma unroll
     for (int j = 0; j < C::FN; ++j) acc[i][j] = typename Traits<C::MODE>::acc_t{};
   const FragAddr<C> ad(id, lane);
-  const int64_t count = stages<C>(Kb);
-  load(0);
-  store(0);
-  load(1);
+#pragma unroll
+  for (int d = 0; d < AHEAD; ++d) load(regs[d], d);
+  store(regs[0], 0);
+  load(regs[0], AHEAD);
   __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   stage_barrier();
-  for (int64_t kt = 0; kt < count; ++kt) {
+  // Stage kt + 1 waits in register set (kt + 1) % AHEAD; kt advances AHEAD stages per pass (the
+  // trailing ones hold zeros), so the sets are compile-time.
+  auto step = [&](auto set_tag, int64_t kt) {
+    constexpr int SET = (decltype(set_tag)::value + 1) % AHEAD;
     const int buf = static_cast<int>(kt & 1);
     Frags<C> f;
     read_stage<C>(lds + buf * C::STAGE, ad, f);
-    store(buf ^ 1);  // stage kt + 1; the buffer's last reads ended before the barrier
-    load(kt + 2);
+    store(regs[SET], buf ^ 1);  // the buffer's last reads ended before the barrier
+    load(regs[SET], kt + 1 + AHEAD);
 #pragma unroll
     for (int i = 0; i < C::FM; ++i)
 #pragma unroll
       for (int j = 0; j < C::FN; ++j) mfma<C::MODE>(acc[i][j], f.a[i], f.b[j]);
     __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     stage_barrier();
+  };
+  for (int64_t kt = 0; kt < count; kt += AHEAD) {
+    step(std::integral_constant<int, 0>{}, kt);
+    if (kt + 1 < count) step(std::integral_constant<int, 1>{}, kt + 1);
+    if (kt + 2 < count) step(std::integral_constant<int, 2>{}, kt + 2);
   }
 }
 
