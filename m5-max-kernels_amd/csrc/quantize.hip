@@ -228,8 +228,10 @@ __global__ __launch_bounds__(kThreads) void quantize_mx_kernel(const uint8_t* __
 
 // MXINT8 codes to BF16 values code * 2^(e - 127): exact (|code| <= 127 fits the BF16
 // significand), 8 elements per thread.  Two matrices, the GEMM's operands, in one launch: the smaller
-// one's threads run beside the larger one's instead of in a launch of their own ([1024, 4096] and
-// [4096, 4096]: 12.0 us against 4.7 + 9.0 us and the gap between them).
+// one's workgroups run beside the larger one's instead of in a launch of their own ([1024, 4096] and
+// [4096, 4096]: 11.2 us against 13.0 us; [1546, 4096] and [14336, 4096]: 29.4 against 31.5 us).  A
+// workgroup holds groups of one matrix only, so the pointers stay in scalar registers: with them
+// chosen per thread the larger pair took 4 us more.
 struct MxMatrix {
   const int8_t* q;
   const uint8_t* s;
@@ -237,14 +239,12 @@ struct MxMatrix {
   int64_t groups;  // of 8 elements
 };
 
-__global__ __launch_bounds__(kThreads) void mx_to_bf16_kernel(MxMatrix first, MxMatrix second) {
-  int64_t t = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
-  MxMatrix a = first;
-  if (t >= first.groups) {
-    t -= first.groups;
-    a = second;
-    if (t >= second.groups) return;
-  }
+__global__ __launch_bounds__(kThreads) void mx_to_bf16_kernel(MxMatrix first, MxMatrix second, int first_blocks) {
+  const int block = blockIdx.x;
+  const bool lead = block < first_blocks;
+  const MxMatrix a = lead ? first : second;
+  const int64_t t = static_cast<int64_t>(lead ? block : block - first_blocks) * kThreads + threadIdx.x;
+  if (t >= a.groups) return;
   const uint2 w = *reinterpret_cast<const uint2*>(a.q + t * 8);
   const int e = static_cast<int>(a.s[t >> 2]) - 127;
   uint32_t out[4];
@@ -260,9 +260,11 @@ __global__ __launch_bounds__(kThreads) void mx_to_bf16_kernel(MxMatrix first, Mx
 }
 
 int launch_mx_to_bf16(const MxMatrix& first, const MxMatrix& second, hipStream_t st, const char* name) {
-  const int64_t blocks = (first.groups + second.groups + kThreads - 1) / kThreads;
+  const int64_t first_blocks = (first.groups + kThreads - 1) / kThreads;
+  const int64_t blocks = first_blocks + (second.groups + kThreads - 1) / kThreads;
   M5K_REQUIRE(blocks <= 0x7FFFFFFF, "%s: input too large", name);
-  mx_to_bf16_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, st>>>(first, second);
+  mx_to_bf16_kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0, st>>>(first, second,
+                                                                                   static_cast<int>(first_blocks));
   return launch_status(name);
 }
 
