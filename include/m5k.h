@@ -210,8 +210,11 @@ int m5k_gemm_schedule_state(void);
  * INT8 results are bit-identical under every tile.  Float results (FP32 sums) are the same bits for
  * tiles 1 to 3, and for tile 0 under every schedule; between these groups and tile 4 the order of the
  * sum differs.  Float rows of under 1 KiB always take tile 0.
+ * max_splits (1..64, more than 1 for I8 and U8 only) offers the split entry points' K ranges too;
+ * *splits receives how many the choice takes (1: no partial sums; tiles 0 and 4 always).
  */
-int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int* tile);
+int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int max_splits, int* tile,
+                       int* splits);
 
 /*
  * Raw INT32 accumulators of the W8A8 GEMM (test hook for bit-exact parity):

@@ -70,20 +70,28 @@ extern "C" int m5k_gemm_schedule_state(void) {
          (off("M5K_GEMM_MIXED_TILES") ? 16 : 0) | (off("M5K_GEMM_NARROW_TILES") ? 32 : 0);
 }
 
-extern "C" int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int* tile) {
+extern "C" int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int max_splits,
+                                  int* tile, int* splits) {
   clear_error();
   const char* name = "m5k_gemm_tile_plan";
-  M5K_REQUIRE(tile != nullptr, "%s: null output", name);
+  M5K_REQUIRE(tile != nullptr && splits != nullptr, "%s: null output", name);
   if (int rc = check_shape(m, n, k, name)) return rc;
   M5K_REQUIRE(cus > 0, "%s: cus must be positive", name);
+  M5K_REQUIRE(max_splits >= 1 && max_splits <= 64, "%s: max_splits=%d outside [1,64]", name, max_splits);
+  int mode, bytes;
   switch (ab_dtype) {
-    case M5K_I8: *tile = plan_tile(I8, m, n, k, cus, aligned != 0).tile; return M5K_OK;
-    case M5K_U8: *tile = plan_tile(F8, m, n, k, cus, aligned != 0).tile; return M5K_OK;
-    case M5K_BF16: *tile = plan_tile(BF16, m, n, 2 * k, cus, aligned != 0).tile; return M5K_OK;
-    case M5K_F16: *tile = plan_tile(F16, m, n, 2 * k, cus, aligned != 0).tile; return M5K_OK;
-    case M5K_F32: *tile = plan_tile(F32, m, n, 4 * k, cus, aligned != 0).tile; return M5K_OK;
+    case M5K_I8: mode = I8, bytes = 1; break;
+    case M5K_U8: mode = F8, bytes = 1; break;
+    case M5K_BF16: mode = BF16, bytes = 2; break;
+    case M5K_F16: mode = F16, bytes = 2; break;
+    case M5K_F32: mode = F32, bytes = 4; break;
     default: set_error("%s: ab_dtype must be I8, U8 (FP8 codes), BF16, F16 or F32", name); return M5K_EINVAL;
   }
+  M5K_REQUIRE(max_splits == 1 || mode == I8 || mode == F8, "%s: only I8 and U8 products split over K", name);
+  const plan::Choice c = plan_tile(mode, m, n, k * bytes, cus, aligned != 0, max_splits);
+  *tile = c.tile;
+  *splits = c.splits;
+  return M5K_OK;
 }
 
 extern "C" int m5k_gemm_set_schedule(int schedule, int* previous) {

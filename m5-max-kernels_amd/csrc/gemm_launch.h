@@ -429,7 +429,7 @@ int launch_ring_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n,
 // fill the CUs needs none, and then no partial sums exist (128 x 4096 x 4096 INT8 with 4 ranges of 256
 // x 64 tiles and the epilogue pass 16.2 us; unsplit 64 x 64 tiles 9.7 us).  The 256-row tiles serve
 // what is left, middle M with a long K: 256 x 128 where their workgroups fit in one round, else 256 x
-// 256 (M 1024, N 5376, K 14336: 84 us with 3 ranges, 94 us unsplit).
+// 256 (M 900, N 5376, K 14336: 86.5 us with 3 ranges, 93.5 us unsplit).
 template <int MODE, int OUT_DT, int BIAS, int GATE, class P>
 int launch_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int64_t kb, const EpiParams& p, int splits,
                   P* workspace, hipStream_t st, const char* name) {
@@ -443,10 +443,9 @@ int launch_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int6
   const int tn = half ? HalfGrid::TN : BN;
   const int64_t wgs_256 = tiles_m * ((n + tn - 1) / tn) * used;
   const double rounds = cus > 0 ? static_cast<double>((wgs_256 + cus - 1) / cus) : 1.0;
-  // Half tiles run short of their share here: 512 x 7168 x 14336 in 2 ranges 82 us, 768 x 5376 x 14336
-  // 69 us, where their time in a mixed launch predicts 62 and 64.
-  const double split_256 = plan::tile256_us(rounds * (half ? 1.25 * kHalfTileCost : 1.0), n, kb / used) +
-                           plan::split_us(m, n, used);
+  // Half tiles take a little more than in a mixed launch (768 x 5376 x 14336 in 2 ranges 69 us).
+  const double split_256 =
+      plan::tile256_us(rounds * (half ? 1.08 * kHalfTileCost : 1.0), n, kb / used) + plan::split_us(m, n, used);
   const double plain_256 = plan::tile256_us(units_256(md16, m, n, cus), n, kb);
   const plan::Choice c = plan_tile(MODE, m, n, kb, cus, true, splits, std::min(split_256, plain_256));
   if ((c.tile == plan::TILE_256 && plain_256 < split_256) || (c.tile != plan::TILE_256 && c.splits == 1))

@@ -74,7 +74,7 @@ inline double tile_us(int tile, int64_t m, int64_t n, int64_t kb, int cus, int s
   return with_stream(us, n, kb) + split_us(m, n, splits);
 }
 
-// `units_256`: the 256-row schedules' time in 256 x 256 tile times.
+// `units_256`: the 256-row schedules' time in 256 x 256 tile times; they stream the weight at 2 MB/us.
 inline double tile256_us(double units_256, int64_t n, int64_t kb) {
   return with_stream(units_256 * (13.0 + 10.0e-3 * static_cast<double>(kb)), n, kb, 2.0e6);
 }

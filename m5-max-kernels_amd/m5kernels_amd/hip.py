@@ -228,12 +228,13 @@ TILES = ("256", "128", "64", "64-deep", "decode")
 
 
 @functools.lru_cache(maxsize=4096)
-def _tile_plan(mode, m, n, k, cus, aligned, forced):
-    """The library's tile for an [m, n, k] product (m5k_gemm_tile_plan; host only), cached per shape
-    and schedule settings `forced`, which the library reads itself."""
-    tile = ctypes.c_int(0)
+def _tile_plan(mode, m, n, k, cus, aligned, forced, max_splits=1):
+    """The library's tile for an [m, n, k] product in at most max_splits K ranges (m5k_gemm_tile_plan;
+    host only), cached per shape and schedule settings `forced`, which the library reads itself."""
+    tile, splits = ctypes.c_int(0), ctypes.c_int(0)
     lib = _lib.load()
-    if lib.m5k_gemm_tile_plan(_PLAN_DTYPES[mode], m, n, k, cus, int(aligned), ctypes.byref(tile)):
+    if lib.m5k_gemm_tile_plan(_PLAN_DTYPES[mode], m, n, k, cus, int(aligned), max_splits, ctypes.byref(tile),
+                              ctypes.byref(splits)):
         raise RuntimeError(lib.m5k_last_error().decode(errors="replace"))
     return TILES[tile.value]
 
@@ -261,7 +262,7 @@ def _i8_schedule(m, n, k, cus, env):
     if env[2]:
         return 1, None  # a schedule forced from the environment runs unsplit, as named
     splits = splitk_plan(m, n, k, cus)
-    if splits > 1 and _tile_plan("int8", m, n, k, cus, True, (None, env)) == "decode":
+    if splits > 1 and _tile_plan("int8", m, n, k, cus, True, (None, env), splits) == "decode":
         splits = 1  # a few rows: the decode tile splits K inside its workgroups
     # The library's mixed and narrow launches refill a partial last round without INT32
     # partials and measured faster wherever both apply; the split-K tail takes the rest.

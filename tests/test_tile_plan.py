@@ -44,8 +44,18 @@ def test_a_forced_schedule_keeps_the_256_row_tiles():
 
 
 def test_argument_checks():
-    lib, tile = _lib.load(), ctypes.c_int(0)
-    assert lib.m5k_gemm_tile_plan(_lib.I8, 0, 4, 4, 256, 1, ctypes.byref(tile)) == 1
-    assert lib.m5k_gemm_tile_plan(_lib.I8, 4, 4, 4, 0, 1, ctypes.byref(tile)) == 1
-    assert lib.m5k_gemm_tile_plan(_lib.I32, 4, 4, 4, 256, 1, ctypes.byref(tile)) == 1
-    assert lib.m5k_gemm_tile_plan(_lib.I8, 4, 4, 4, 256, 1, None) == 1
+    lib, tile, splits = _lib.load(), ctypes.c_int(0), ctypes.c_int(0)
+    out = ctypes.byref(tile), ctypes.byref(splits)
+    assert lib.m5k_gemm_tile_plan(_lib.I8, 4, 4, 4, 256, 1, 1, *out) == 0
+    assert lib.m5k_gemm_tile_plan(_lib.I8, 0, 4, 4, 256, 1, 1, *out) == 1
+    assert lib.m5k_gemm_tile_plan(_lib.I8, 4, 4, 4, 0, 1, 1, *out) == 1
+    assert lib.m5k_gemm_tile_plan(_lib.I32, 4, 4, 4, 256, 1, 1, *out) == 1
+    assert lib.m5k_gemm_tile_plan(_lib.I8, 4, 4, 4, 256, 1, 65, *out) == 1
+    assert lib.m5k_gemm_tile_plan(_lib.BF16, 4, 4, 4, 256, 1, 2, *out) == 1
+    assert lib.m5k_gemm_tile_plan(_lib.I8, 4, 4, 4, 256, 1, 1, None, None) == 1
+
+
+def test_a_long_k_splits_where_decode_would_leave_cus_idle():
+    # 30 x 2048 x 16384: 128 decode workgroups of 32 rows took 24 us, K ranges of ring tiles 14 us.
+    assert hip._tile_plan.__wrapped__("int8", 30, 2048, 16384, 256, True, None, 16) != "decode"
+    assert hip._tile_plan.__wrapped__("int8", 1, 4096, 4096, 256, True, None, 4) == "decode"
