@@ -10,7 +10,7 @@ Differences that follow from the platform, not the contract:
 
 * ``tile=(TM, TN, groups, swizzle)`` names an Apple threadgroup tiling.  It is
   unpacked (so malformed tuples fail as in the reference) but the MI355X kernel
-  always uses its own 256x256 MFMA tile with an XCD-aware raster.
+  chooses its own MFMA tile from the sizes (csrc/gemm_plan.h), with an XCD-aware raster.
 * ``tag`` only specialized the Metal kernel name; it is accepted and ignored.
 * ``mode="mxint8"`` GEMM expands both operands exactly to BF16 (codes times their block
   scale) and runs the BF16 MFMA GEMM with FP32 accumulation.
@@ -107,22 +107,20 @@ def splitk_plan(m, n, k, cus=256, skinny=True):
     so splits also stay below K / (2 M).  (Measured on MI355X over M 16..512 and H3 widths:
     within ~10% of the best split count, 1.4-3.7x faster than one workgroup per tile.)
 
-    It first tries the library's narrower split tiles, which m5k_gemm_i8_splitk uses whenever
-    ceil(M / 256) * ceil(N / width) * splits fits in one round of `cus` workgroups: 256 x 64
-    (K <= 8192), then 256 x 128.  Fewer K ranges then fill the chip (measured 1.4-1.6x faster
-    at K 4096-5376 with 64-wide tiles, 1.15-1.23x at N 14336 or K 14336-16384 with 128-wide
-    ones, 1.1-1.45x at M 384-1024).  Above M = 768, with at least 32 tiles of 256 x 256, the
-    plain launch (the library's mixed or narrow tiles) measured faster than any split (M 1024:
-    44.8 against 57.6 us at N = K = 5376, 35.5 against 37.2 us at N = K = 4096), so no split is
-    planned there, unless K is long and the tiles fill under 3/8 of the CUs (then the chip takes
-    cus // tiles K ranges); narrow outputs (N 32-96) keep the split, their few tiles leaving most
-    CUs idle.
-    skinny=False plans without the 256 x 64 tile (the FP8 split, m5k_gemm_f8_splitk)."""
+    Ranges are counted in the narrowest width of column that lets M / 256 rows of them fill at most
+    one round of `cus` workgroups: 64 columns (K <= 8192), then 128, then 256.  The library launches
+    that many on its 256-row tiles (128 columns wide where they fit in one round), or fewer or none
+    on 128- and 64-row tiles where its planner expects those to be faster.  Above M = 768, with at
+    least 32 tiles of 256 x 256, the unsplit launch (the library's mixed or narrow tiles) measured
+    faster than any split (M 1024: 44.8 against 57.6 us at N = K = 5376), so no split is planned
+    there, unless K is long and the tiles fill under 3/8 of the CUs (then the chip takes cus // tiles
+    K ranges); narrow outputs (N 32-96) keep the split, their few tiles leaving most CUs idle.
+    skinny=False plans without the 64-column ranges (the FP8 split, m5k_gemm_f8_splitk)."""
     slabs = -(-k // 64)
     if m > 768 and -(-m // 256) * -(-n // 256) >= 32:
         # One partial round that even the mixed launch's half tiles fill to under 3/4, over a
-        # long K: whole-tile K ranges fill the chip instead (M 1024: 84 tiles at N 5376, K 14336
-        # ran 94.0 -> 84.3 us with 3 ranges; 64 at N 4096, K 16384 97.7 -> 77.5 us with 4; at
+        # long K: whole-tile K ranges fill the chip instead (M 900: 84 tiles at N 5376, K 14336
+        # ran 93.5 -> 86.5 us with 3 ranges; 64 at N 4096, K 16384 97.7 -> 77.5 us with 4; at
         # K 5376, or M 1536 and up, the plain and mixed launches stayed ahead).
         tiles = -(-m // 256) * -(-n // 256)
         if k >= 8192 and 2 * tiles <= 3 * cus // 4:

@@ -5,8 +5,8 @@ function names, signatures, defaults and exception types.  Boundaries: BF16 proj
 RMS / gamma / RoPE, BF16 head-major output [heads, M, 128]; no BF16 norm intermediate.
 
 ``tile=(TM, TN, groups, swizzle)`` and ``threads`` are validated as in the reference (they
-named Apple threadgroup shapes); the gfx950 kernels always use a 256-row x 2-head MFMA tile
-and 16-lane groups per (row, head).
+named Apple threadgroup shapes); the gfx950 kernels use 256-row x 2-head or 128-row x one-head
+MFMA tiles, whichever the plain GEMM would, and 16-lane groups per (row, head).
 """
 
 from __future__ import annotations
