@@ -107,8 +107,7 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
 def load_fast():
     """The native front of quantize() and gemm() (binding/fast_ops.cpp), linked against libm5k.so, or
     None where the libraries have not been built.  One that does not load (left from an older build)
-    warns: the same kernels then run with the checks in Python, and this package still imports, so that
-    it can be built again."""
+    warns: the same kernels then run with the checks in Python."""
     if not (FAST_PATH.exists() and LIB_PATH.exists()) or _current_raw_stream is None:
         return None
     spec = importlib.util.spec_from_file_location("m5k_fast", FAST_PATH)

@@ -561,6 +561,36 @@ def gemm_i8_accumulators(a, b):
     return acc
 
 
-_fast = _lib.load_fast()
-if _fast is not None:
-    _fast.bind(_lib._current_raw_stream, _native_splits)
+class _NativeFront:
+    """The native front (binding/fast_ops.cpp), loaded by the first call that it is offered; a call that
+    it does not take, or every call where it is not built, gets None.  Importing this package maps no
+    library: the dynamic loader keeps a mapped file for its path, so a process that imports, builds and
+    runs would otherwise go on with the library that its build replaced."""
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._module = None
+        self._done = False
+
+    def _load(self):
+        global _fast
+        with self._lock:
+            if not self._done and _lib.LIB_PATH.exists():
+                self._module = _lib.load_fast()
+                if self._module is not None:
+                    self._module.bind(_lib._current_raw_stream, _native_splits)
+                self._done = True
+                if _fast is self:
+                    _fast = self._module
+        return self._module
+
+    def quantize(self, *args):
+        module = self._load()
+        return None if module is None else module.quantize(*args)
+
+    def gemm(self, *args):
+        module = self._load()
+        return None if module is None else module.gemm(*args)
+
+
+_fast = _NativeFront()
