@@ -70,6 +70,7 @@ extern "C" {
 const char* m5k_last_error(void);
 
 /* ABI version (major*100 + minor). */
+#define M5K_ABI_VERSION 100
 int m5k_abi_version(void);
 
 /*

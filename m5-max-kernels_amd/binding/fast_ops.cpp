@@ -278,4 +278,14 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "m5k_fast", nullptr, -1, methods, n
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit_m5k_fast() { return PyModule_Create(&module); }
+// abi_version and torch_version: what this file was compiled for, compared before the first call
+// (_lib.load_fast).
+PyMODINIT_FUNC PyInit_m5k_fast() {
+  PyObject* m = PyModule_Create(&module);
+  if (m != nullptr && (PyModule_AddIntConstant(m, "abi_version", M5K_ABI_VERSION) != 0 ||
+                       PyModule_AddStringConstant(m, "torch_version", M5K_TORCH_VERSION) != 0)) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

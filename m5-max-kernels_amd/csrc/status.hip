@@ -46,4 +46,4 @@ int device_cus() {
 
 extern "C" const char* m5k_last_error(void) { return m5k::g_error; }
 
-extern "C" int m5k_abi_version(void) { return 100; }
+extern "C" int m5k_abi_version(void) { return M5K_ABI_VERSION; }

@@ -106,8 +106,9 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
 
 def load_fast():
     """The native front of quantize() and gemm() (binding/fast_ops.cpp), linked against libm5k.so, or
-    None where the libraries have not been built.  One that does not load (left from an older build)
-    warns: the same kernels then run with the checks in Python."""
+    None where the libraries have not been built.  One that does not load, or that was compiled for
+    another C ABI or another torch (left from an older build), warns: the same kernels then run with
+    the checks in Python."""
     if not (FAST_PATH.exists() and LIB_PATH.exists()) or _current_raw_stream is None:
         return None
     spec = importlib.util.spec_from_file_location("m5k_fast", FAST_PATH)
@@ -116,6 +117,12 @@ def load_fast():
         spec.loader.exec_module(module)
     except ImportError as e:
         warnings.warn(f"{FAST_PATH.name} does not load ({e}); build the package again", RuntimeWarning)
+        return None
+    built_for = getattr(module, "abi_version", None), getattr(module, "torch_version", None)
+    running = load().m5k_abi_version(), torch.__version__
+    if built_for != running:
+        warnings.warn(f"{FAST_PATH.name} was compiled for (C ABI, torch) {built_for}, this process has {running}; "
+                      "build the package again", RuntimeWarning)
         return None
     return module
 

@@ -81,11 +81,10 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     LIB_PATH.parent.mkdir(parents=True, exist_ok=True)
     srcs = sources()
     jobs = jobs or min(len(srcs), max(1, min(8, os.cpu_count() or 1)))
-    fast_obj = BUILD_DIR / "fast_ops.o"
     with ThreadPoolExecutor(max_workers=jobs) as pool:
-        fast = pool.submit(_compile_fast, fast_obj, force)
+        fast = pool.submit(_compile_fast, force)
         objs = list(pool.map(lambda s: _compile(s, force), srcs))
-        fast.result()
+        fast_obj = fast.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -99,21 +98,24 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     return LIB_PATH
 
 
-def _compile_fast(obj: Path, force: bool) -> None:
+def _compile_fast(force: bool) -> Path:
     """The native front of quantize() and gemm(): host code against torch's headers."""
     import torch
     from torch.utils.cpp_extension import include_paths
 
+    obj = BUILD_DIR / f"fast_ops-{torch.__version__}.o"  # an object of another torch is no object of this one
     newest_dep = max(p.stat().st_mtime for p in [FAST_SRC, *INCLUDE.glob("*.h")])
     if not force and obj.exists() and obj.stat().st_mtime >= newest_dep:
-        return
+        return obj
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{INCLUDE}",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DM5K_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}",
            f"-I{sysconfig.get_paths()['include']}", *(f"-isystem{p}" for p in include_paths()),
            "-c", str(FAST_SRC), "-o", str(obj)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"compile of {FAST_SRC.name} failed:\n{proc.stderr[-4000:]}")
+    return obj
 
 
 def _link_fast(obj: Path) -> None:

@@ -44,3 +44,30 @@ def test_without_the_native_front_the_python_one_takes_the_call(monkeypatch):
     with pytest.raises(ValueError, match="unknown quantization mode"):
         quantize(torch.zeros(2, 2), "int9")
     assert hip._fast is None
+
+
+@pytest.fixture
+def older_abi(monkeypatch):
+    """The loaded library, with another ABI version than m5k_fast.so was compiled for."""
+    lib = _lib.load()
+
+    class Other:
+        m5k_abi_version = staticmethod(lambda: lib.m5k_abi_version() + 100)
+
+    monkeypatch.setattr(_lib, "load", lambda: Other)
+
+
+def test_a_front_of_another_abi_is_refused(older_abi):
+    with pytest.warns(RuntimeWarning, match="compiled for"):
+        assert _lib.load_fast() is None
+
+
+def test_a_front_of_another_torch_is_refused(monkeypatch):
+    monkeypatch.setattr(torch, "__version__", "0.0.1")
+    with pytest.warns(RuntimeWarning, match="compiled for"):
+        assert _lib.load_fast() is None
+
+
+def test_the_built_front_matches_the_library():
+    front = _lib.load_fast()
+    assert front.abi_version == _lib.load().m5k_abi_version() and front.torch_version == torch.__version__
