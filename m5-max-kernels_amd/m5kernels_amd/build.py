@@ -2,8 +2,10 @@
 
 Every translation unit under ``csrc/`` is compiled to an object under ``_build/``
 (in parallel), then linked into ``lib/libm5k.so`` next to this package.  The measurement
-kernels under ``diag/`` (bench.py's MFMA ceiling) go into ``lib/libm5k_diag.so``, the native front of quantize() and gemm() under ``binding/`` (host code, against
-torch's headers) into ``lib/m5k_fast.so``.  Flags:
+kernels under ``diag/`` (bench.py's MFMA ceiling) go into ``lib/libm5k_diag.so``, the native
+front of quantize() and gemm() under ``binding/`` (host code, against torch's headers) into
+``lib/m5k_fast.so``; where those headers are missing the other two are built all the same.
+Flags:
 
 * ``--offload-arch=gfx950`` only: MI355X is the single target.
 * ``-ffp-contract=off``: no FMA contraction, so FP32 epilogues and normalization keep
@@ -20,6 +22,7 @@ import shutil
 import subprocess
 import sys
 import sysconfig
+import warnings
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -84,34 +87,52 @@ def build(force: bool = True, jobs: int | None = None, verbose: bool = False) ->
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         fast = pool.submit(_compile_fast, force)
         objs = list(pool.map(lambda s: _compile(s, force), srcs))
-        fast_obj = fast.result()
     tmp = LIB_PATH.with_suffix(".so.tmp")
     cmd = [hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"link of libm5k.so failed:\n{proc.stderr[-4000:]}")
     os.replace(tmp, LIB_PATH)
-    _link_fast(fast_obj)
     build_diag()
+    # The library stands by itself; the front is built beside it, and an older one does not stay there.
+    FAST_PATH.unlink(missing_ok=True)
+    if (fast_obj := fast.result()) is not None:
+        _link_fast(fast_obj)
     if verbose:
         print(f"built {LIB_PATH} from {len(srcs)} sources, and {DIAG_LIB_PATH}", file=sys.stderr)
     return LIB_PATH
 
 
-def _compile_fast(force: bool) -> Path:
-    """The native front of quantize() and gemm(): host code against torch's headers."""
-    import torch
-    from torch.utils.cpp_extension import include_paths
+def _front_includes() -> list[str]:
+    """Include folders of the native front, or none where g++, Python's or torch's headers are not
+    installed: libm5k.so needs none of them."""
+    try:
+        from torch.utils.cpp_extension import include_paths
+    except ImportError:  # setuptools, which torch's extension builder imports
+        return []
+    python, folders = sysconfig.get_paths()["include"], include_paths()
+    if not (shutil.which("g++") and (Path(python) / "Python.h").exists()
+            and any((Path(p) / "torch" / "extension.h").exists() for p in folders)):
+        return []
+    return [f"-I{python}", *(f"-isystem{p}" for p in folders)]
 
+
+def _compile_fast(force: bool) -> Path | None:
+    """The native front of quantize() and gemm(): host code against torch's headers (None without
+    them: quantize() and gemm() then run their checks in Python)."""
+    import torch
+
+    includes = _front_includes()
+    if not includes:
+        warnings.warn("g++, Python.h or torch's headers are missing: m5k_fast.so is not built", RuntimeWarning)
+        return None
     obj = BUILD_DIR / f"fast_ops-{torch.__version__}.o"  # an object of another torch is no object of this one
     newest_dep = max(p.stat().st_mtime for p in [FAST_SRC, *INCLUDE.glob("*.h")])
     if not force and obj.exists() and obj.stat().st_mtime >= newest_dep:
         return obj
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
-           f'-DM5K_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}",
-           f"-I{sysconfig.get_paths()['include']}", *(f"-isystem{p}" for p in include_paths()),
-           "-c", str(FAST_SRC), "-o", str(obj)]
+           f'-DM5K_TORCH_VERSION="{torch.__version__}"', f"-I{INCLUDE}", *includes, "-c", str(FAST_SRC), "-o", str(obj)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"compile of {FAST_SRC.name} failed:\n{proc.stderr[-4000:]}")
