@@ -129,12 +129,14 @@ int m5k_gemm_i8(const int8_t* a, const int8_t* b, int64_t m, int64_t n, int64_t 
 /*
  * The same W8A8 linear as m5k_gemm_i8 for short M: each output tile may be split over up to
  * `splits` contiguous ranges of K (1..64).  The library takes the tile and the number of ranges
- * that it expects to be fastest; with one range it is m5k_gemm_i8's launch and the workspace stays
- * untouched.  Otherwise the raw INT32 partial tiles go to workspace[splits][m][n] (int32,
- * caller-owned, at least splits*m*n elements), and a second kernel sums them in split order and
- * applies the identical epilogue.  INT32 sums are exact, so c is bit-identical to m5k_gemm_i8's.  Needs k % 16 == 0 and 16-byte aligned a/b (any operand size).  Same
- * contract as metal.gemm(a, b, "int8", ...) (src/m5kernels/metal.py:158-269); the split is
- * this library's schedule for few-tile shapes (one or two 256-row tile rows).
+ * that it expects to be fastest (m5k_gemm_split_plan reports them; m5k_gemm_set_exact_splits makes
+ * it run `splits`); with one range it is m5k_gemm_i8's launch and the workspace stays untouched.
+ * Otherwise the raw INT32 partial tiles go to workspace[splits][m][n] (int32, caller-owned, at
+ * least splits*m*n elements), and a second kernel sums them in split order and applies the
+ * identical epilogue.  INT32 sums are exact, so c is bit-identical to m5k_gemm_i8's.  Needs
+ * k % 16 == 0 and 16-byte aligned a/b (any operand size).  Same contract as
+ * metal.gemm(a, b, "int8", ...) (src/m5kernels/metal.py:158-269); the split is this library's
+ * schedule for outputs whose tiles leave CUs idle (few rows, or few columns).
  */
 int m5k_gemm_i8_splitk(const int8_t* a, const int8_t* b, int64_t m, int64_t n, int64_t k,
                        const float* a_scales, const float* b_scales, void* c, int c_dtype,
@@ -195,7 +197,8 @@ int m5k_gemm_set_schedule(int schedule, int* previous);
 /*
  * What decides the calling thread's schedules besides the shape, as one value (a key for host-side
  * plan caches; no counterpart in the reference): bits 0-2 the thread's forced schedule + 1, bit 3 a
- * schedule in M5K_GEMM_SCHEDULE, bits 4 and 5 M5K_GEMM_MIXED_TILES=0 and M5K_GEMM_NARROW_TILES=0.
+ * schedule in M5K_GEMM_SCHEDULE, bits 4 and 5 M5K_GEMM_MIXED_TILES=0 and M5K_GEMM_NARROW_TILES=0,
+ * bit 6 the thread's exact K ranges (m5k_gemm_set_exact_splits).
  */
 int m5k_gemm_schedule_state(void);
 
@@ -211,11 +214,30 @@ int m5k_gemm_schedule_state(void);
  * INT8 results are bit-identical under every tile.  Float results (FP32 sums) are the same bits for
  * tiles 1 to 3, and for tile 0 under every schedule; between these groups and tile 4 the order of the
  * sum differs.  Float rows of under 1 KiB always take tile 0.
- * max_splits (1..64, more than 1 for I8 and U8 only) offers the split entry points' K ranges too;
- * *splits receives how many the choice takes (1: no partial sums; tiles 0 and 4 always).
+ * max_splits (1..64, more than 1 for I8 and U8 only) offers K ranges of tiles 1 to 3 too; *splits
+ * receives how many the choice takes (1: no partial sums; tiles 0 and 4 always).  K ranges of
+ * 256-row tiles are not weighed here: m5k_gemm_split_plan has the split entry points' whole choice.
  */
 int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int max_splits, int* tile,
                        int* splits);
+
+/*
+ * What a split entry point (m5k_gemm_i8_splitk[_noalloc]: I8; m5k_gemm_f8_splitk: U8) launches on a
+ * device of `cus` compute units for `splits` (1..64), under the calling thread's settings (host only,
+ * launches nothing; no counterpart in the reference).  *ranges receives the K ranges that run; 1: the
+ * unsplit launch, which leaves the workspace alone.  *tile receives the tile as in m5k_gemm_tile_plan,
+ * with 5 for 256 x 128 tiles; tile 0 with ranges above 1 is 256 x 256.
+ */
+int m5k_gemm_split_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int splits, int* tile, int* ranges);
+
+/*
+ * Whether the split entry points of the calling host thread run exactly the K ranges that a call names
+ * (on != 0; fewer only where a range would be empty), or up to as many as the library expects to pay
+ * (0, the default).  A forced schedule (m5k_gemm_set_schedule) does the same, on its 256-row tiles.
+ * *previous (may be NULL) receives the earlier setting.  No counterpart in the reference: the harness
+ * tuner times split counts through it, and tests run each split kernel.
+ */
+int m5k_gemm_set_exact_splits(int on, int* previous);
 
 /*
  * Raw INT32 accumulators of the W8A8 GEMM (test hook for bit-exact parity):

@@ -67,7 +67,8 @@ extern "C" int m5k_gemm_schedule_state(void) {
   };
   const char* forced = std::getenv("M5K_GEMM_SCHEDULE");
   return (g_thread_schedule + 1) | (forced != nullptr && forced[0] != '\0' ? 8 : 0) |
-         (off("M5K_GEMM_MIXED_TILES") ? 16 : 0) | (off("M5K_GEMM_NARROW_TILES") ? 32 : 0);
+         (off("M5K_GEMM_MIXED_TILES") ? 16 : 0) | (off("M5K_GEMM_NARROW_TILES") ? 32 : 0) |
+         (g_thread_exact_splits ? 64 : 0);
 }
 
 extern "C" int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int aligned, int max_splits,
@@ -91,6 +92,29 @@ extern "C" int m5k_gemm_tile_plan(int ab_dtype, int64_t m, int64_t n, int64_t k,
   const plan::Choice c = plan_tile(mode, m, n, k * bytes, cus, aligned != 0, max_splits);
   *tile = c.tile;
   *splits = c.splits;
+  return M5K_OK;
+}
+
+extern "C" int m5k_gemm_split_plan(int ab_dtype, int64_t m, int64_t n, int64_t k, int cus, int splits, int* tile,
+                                   int* ranges) {
+  clear_error();
+  const char* name = "m5k_gemm_split_plan";
+  M5K_REQUIRE(tile != nullptr && ranges != nullptr, "%s: null output", name);
+  if (int rc = check_shape(m, n, k, name)) return rc;
+  M5K_REQUIRE(cus > 0, "%s: cus must be positive", name);
+  M5K_REQUIRE(splits >= 1 && splits <= 64, "%s: splits=%d outside [1,64]", name, splits);
+  M5K_REQUIRE(ab_dtype == M5K_I8 || ab_dtype == M5K_U8, "%s: only I8 and U8 products split over K", name);
+  const int mode = ab_dtype == M5K_I8 ? I8 : F8;
+  const SplitPlan c = plan_split(mode, m, n, k, cus, splits);
+  *ranges = c.ranges;
+  *tile = c.ranges > 1 ? c.tile : plan_tile(mode, m, n, k, cus, true).tile;
+  return M5K_OK;
+}
+
+extern "C" int m5k_gemm_set_exact_splits(int on, int* previous) {
+  clear_error();
+  if (previous) *previous = g_thread_exact_splits;
+  g_thread_exact_splits = on != 0;
   return M5K_OK;
 }
 

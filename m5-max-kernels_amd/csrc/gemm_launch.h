@@ -159,6 +159,10 @@ enum Schedule { SCHED_PLAIN = 0, SCHED_MIXED = 1, SCHED_NARROW = 2, SCHED_QUAD =
 // 16 x 16 modes and quad to W8A8; the other modes run plain in their place.
 inline thread_local int g_thread_schedule = -1;
 
+// The split entry points of this host thread run as many K ranges as a call names, not up to as many
+// (m5k_gemm_set_exact_splits: the harness tuner, and tests of the split kernels).
+inline thread_local bool g_thread_exact_splits = false;
+
 inline int forced_schedule(bool md16, bool i8, int64_t m, int64_t n, int cus, int64_t& full) {
   int which = g_thread_schedule;
   if (which < 0) {
@@ -425,33 +429,72 @@ int launch_ring_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n,
   return launch_status(name);
 }
 
-// At most `splits` K ranges per tile, as many as the planner expects to pay: a tile small enough to
-// fill the CUs needs none, and then no partial sums exist (128 x 4096 x 4096 INT8 with 4 ranges of 256
-// x 64 tiles and the epilogue pass 16.2 us; unsplit 64 x 64 tiles 9.7 us).  The 256-row tiles serve
-// what is left, middle M with a long K: 256 x 128 where their workgroups fit in one round, else 256 x
-// 256 (M 900, N 5376, K 14336: 86.5 us with 3 ranges, 93.5 us unsplit).
-template <int MODE, int OUT_DT, int BIAS, int GATE, class P>
-int launch_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int64_t kb, const EpiParams& p, int splits,
-                  P* workspace, hipStream_t st, const char* name) {
-  constexpr bool md16 = MODE != F8;  // the narrow schedule's modes
-  const int64_t kt_total = k_stages(kb);
-  const int64_t per = (kt_total + splits - 1) / splits;
-  int used = static_cast<int>((kt_total + per - 1) / per);  // no empty split
-  const int cus = device_cus();
+// K bytes of a main-loop stage: the ranges are whole stages.
+constexpr int64_t stage_bytes(int mode, int tile) {
+  return tile == plan::TILE_64_DEEP || (mode == F8 && (tile == plan::TILE_128 || tile == plan::TILE_64)) ? 2 * BKB : BKB;
+}
+template <int MODE>
+constexpr bool ring_stages_agree() {
+  using R = RingTiles<MODE>;
+  return R::T128::STAGE_K == stage_bytes(MODE, plan::TILE_128) && R::T64::STAGE_K == stage_bytes(MODE, plan::TILE_64) &&
+         R::Deep::STAGE_K == stage_bytes(MODE, plan::TILE_64_DEEP);
+}
+static_assert(ring_stages_agree<I8>() && ring_stages_agree<F8>(), "K ranges are counted as they are launched");
+
+// Ranges of a row of kb bytes in at most `splits` of equally many stages: none is empty.
+inline int used_ranges(int mode, int tile, int64_t kb, int splits) {
+  const int64_t total = plan::ceil_div(kb, stage_bytes(mode, tile)), per = plan::ceil_div(total, splits);
+  return static_cast<int>(plan::ceil_div(total, per));
+}
+
+struct SplitPlan {
+  int tile;    // plan::Tile
+  int splits;  // K ranges asked of the launch
+  int ranges;  // and those that run; 1: the unsplit launch, with its own choice of tile
+};
+
+// The launch of a split entry point.  At most `splits` K ranges per tile, as many as the planner expects
+// to pay: a tile small enough to fill the CUs needs none, and then no partial sums exist (128 x 4096 x
+// 4096 INT8 with 4 ranges of 256 x 64 tiles and the epilogue pass 16.2 us; unsplit 64 x 64 tiles 9.7
+// us).  The 256-row tiles serve what is left, middle M with a long K: 256 x 128 where their workgroups
+// fit in one round, else 256 x 256 (M 900, N 5376, K 14336: 86.5 us with 3 ranges, 93.5 us unsplit).
+// With the thread's exact setting, or under a forced schedule, the call's count itself runs (fewer only
+// where ranges would be empty), on that schedule's 256-row tiles or on the best tile for that count.
+inline SplitPlan plan_split(int mode, int64_t m, int64_t n, int64_t kb, int cus, int splits) {
+  const bool md16 = mode != F8;  // the narrow schedule's modes
+  const int used = used_ranges(mode, plan::TILE_256, kb, splits);
   const int64_t tiles_m = (m + BM - 1) / BM;
   const bool half = cus > 0 && tiles_m * ((n + HalfGrid::TN - 1) / HalfGrid::TN) * used <= static_cast<int64_t>(cus);
   const int tn = half ? HalfGrid::TN : BN;
-  const int64_t wgs_256 = tiles_m * ((n + tn - 1) / tn) * used;
-  const double rounds = cus > 0 ? static_cast<double>((wgs_256 + cus - 1) / cus) : 1.0;
+  const int64_t wgs = tiles_m * ((n + tn - 1) / tn) * used;
+  const double rounds = cus > 0 ? static_cast<double>((wgs + cus - 1) / cus) : 1.0;
   // Half tiles take a little more than in a mixed launch (768 x 5376 x 14336 in 2 ranges 69 us).
   const double split_256 =
       plan::tile256_us(rounds * (half ? 1.08 * kHalfTileCost : 1.0), n, kb / used) + plan::split_us(m, n, used);
-  const double plain_256 = plan::tile256_us(units_256(md16, m, n, cus), n, kb);
-  const plan::Choice c = plan_tile(MODE, m, n, kb, cus, true, splits, std::min(split_256, plain_256));
-  if ((c.tile == plan::TILE_256 && plain_256 < split_256) || (c.tile != plan::TILE_256 && c.splits == 1))
+  const SplitPlan rows_256{half ? plan::TILE_256_HALF : plan::TILE_256, splits, used};
+  int64_t full = -1;
+  if (forced_schedule(md16, mode == I8, m, n, cus, full) >= 0) return rows_256;
+  plan::Choice c;
+  if (g_thread_exact_splits) {
+    if (splits == 1 || cus <= 0) return rows_256;
+    c = plan::choose(m, n, kb, cus, true, splits, split_256, splits);
+    if (c.tile == plan::TILE_256) return rows_256;
+  } else {
+    const double plain_256 = plan::tile256_us(units_256(md16, m, n, cus), n, kb);
+    c = plan_tile(mode, m, n, kb, cus, true, splits, std::min(split_256, plain_256));
+    if (c.tile == plan::TILE_256) return plain_256 < split_256 ? SplitPlan{plan::TILE_256, 1, 1} : rows_256;
+  }
+  return SplitPlan{c.tile, c.splits, used_ranges(mode, c.tile, kb, c.splits)};
+}
+
+template <int MODE, int OUT_DT, int BIAS, int GATE, class P>
+int launch_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int64_t kb, const EpiParams& p, int splits,
+                  P* workspace, hipStream_t st, const char* name) {
+  const SplitPlan c = plan_split(MODE, m, n, kb, device_cus(), splits);
+  if (c.ranges == 1)
     return launch<MODE, OUT_DT, BIAS, GATE, false>(A, B, m, n, kb / Traits<MODE>::elem_bytes, p, st, name);
   using R = RingTiles<MODE>;
-  int rc = M5K_OK;
+  int used = c.ranges, rc = M5K_OK;
   if (c.tile == plan::TILE_128) {
     rc = launch_ring_splitk<typename R::T128>(A, B, m, n, kb, c.splits, workspace, used, st, name);
   } else if (c.tile == plan::TILE_64) {
@@ -459,6 +502,10 @@ int launch_splitk(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int6
   } else if (c.tile == plan::TILE_64_DEEP) {
     rc = launch_ring_splitk<typename R::Deep>(A, B, m, n, kb, c.splits, workspace, used, st, name);
   } else {
+    const bool half = c.tile == plan::TILE_256_HALF;
+    const int tn = half ? HalfGrid::TN : BN;
+    const int64_t per = plan::ceil_div(k_stages(kb), c.splits);
+    const int64_t wgs_256 = ((m + BM - 1) / BM) * ((n + tn - 1) / tn) * used;
     M5K_REQUIRE(wgs_256 <= 0x7FFFFFFF, "%s: too many workgroups", name);
     const dim3 wgs(static_cast<unsigned>(wgs_256)), block(KernelGrid::THREADS);
     if (half)

@@ -26,7 +26,8 @@ namespace m5k {
 namespace gemm {
 namespace plan {
 
-enum Tile { TILE_256 = 0, TILE_128 = 1, TILE_64 = 2, TILE_64_DEEP = 3, TILE_DECODE = 4 };
+// TILE_256_HALF: 256 x 128 tiles, a form of the K ranges only.
+enum Tile { TILE_256 = 0, TILE_128 = 1, TILE_64 = 2, TILE_64_DEEP = 3, TILE_DECODE = 4, TILE_256_HALF = 5 };
 
 struct Choice {
   int tile;
@@ -79,23 +80,26 @@ inline double tile256_us(double units_256, int64_t n, int64_t kb) {
   return with_stream(units_256 * (13.0 + 10.0e-3 * static_cast<double>(kb)), n, kb, 2.0e6);
 }
 
-// The fastest tile of an [m, n] output with rows of kb bytes and at most max_splits K ranges, or
+// The fastest tile of an [m, n] output with rows of kb bytes and min_splits to max_splits K ranges, or
 // {TILE_256, 1} where none is 5% faster than `limit_us` (the 256-row schedules' time): near the line
 // the predictions err either way.
 // Unaligned operands have the two shallow rings only.
-inline Choice choose(int64_t m, int64_t n, int64_t kb, int cus, bool aligned, int max_splits, double limit_us) {
+inline Choice choose(int64_t m, int64_t n, int64_t kb, int cus, bool aligned, int max_splits, double limit_us,
+                     int min_splits = 1) {
   Choice best{TILE_256, 1, 0.95 * limit_us};
   auto offer = [&](int tile, int splits) {
     const double us = tile_us(tile, m, n, kb, cus, splits);
     if (us < best.us) best = Choice{tile, splits, us};
   };
-  offer(TILE_128, 1);
-  offer(TILE_64, 1);
-  if (!aligned) return best;
-  offer(TILE_64_DEEP, 1);
-  if (m <= 32) offer(TILE_DECODE, 1);
+  if (min_splits == 1) {
+    offer(TILE_128, 1);
+    offer(TILE_64, 1);
+    if (!aligned) return best;
+    offer(TILE_64_DEEP, 1);
+    if (m <= 32) offer(TILE_DECODE, 1);
+  }
   // K ranges of at least 1 KiB.
-  for (int s = 2; s <= max_splits && kb / s >= 1024; ++s) {
+  for (int s = std::max(2, min_splits); s <= max_splits && kb / s >= 1024; ++s) {
     offer(TILE_128, s);
     offer(TILE_64, s);
     offer(TILE_64_DEEP, s);

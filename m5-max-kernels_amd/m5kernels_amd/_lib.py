@@ -59,6 +59,8 @@ SIGNATURES = {
     "m5k_gemm_tile_plan": [_i32, _i64, _i64, _i64, _i32, _i32, _i32, _p, _p],
     "m5k_gemm_set_schedule": [_i32, _p],
     "m5k_gemm_schedule_state": [],
+    "m5k_gemm_split_plan": [_i32, _i64, _i64, _i64, _i32, _i32, _p, _p],
+    "m5k_gemm_set_exact_splits": [_i32, _p],
     "m5k_gemm_i8_splitk": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p, _p, _p, _p, _p, _i32, _p, _i64, _p],
     "m5k_gemm_i8_splitk_noalloc": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p, _p, _p, _p, _p, _i32, _p],
     "m5k_gemm_f8": [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i32, _p],

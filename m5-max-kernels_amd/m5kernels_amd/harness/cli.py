@@ -49,7 +49,7 @@ class Launch:
     """One gfx950 GEMM launch choice; None fields keep the library's plan."""
 
     schedule: str | None = None  # "plain" | "mixed" | "narrow" | "quad"
-    splits: int | None = None  # W8A8 split-K count (1 = no split)
+    splits: int | None = None  # W8A8 K ranges that run (1 = no split)
 
     def record(self):
         return {"schedule": self.schedule or "auto", "splits": self.splits or "auto"}

@@ -180,11 +180,12 @@ _SCHEDULE_CODES = {name: i for i, name in enumerate(SCHEDULES)}
 def launch_override(schedule=None, splits=None):
     """Fix the gfx950 GEMM launch for the calls this thread makes inside the block: `schedule`
     ("plain", "mixed", "narrow" or "quad"; set in the library for this host thread with
-    m5k_gemm_set_schedule) and, for the W8A8 linear, the largest split-K count `splits` (1: no split;
-    the library may take fewer K ranges; the INT32 partials are exact, so every choice gives the same
-    bits).  A forced schedule with
-    `splits` None runs unsplit: the launch timed is the one named.  None keeps the library's own
-    plan.  These are the knobs the harness tuner searches; both settings are thread-local."""
+    m5k_gemm_set_schedule) and, for the W8A8 linear, the number of K ranges `splits` (1: no split; as
+    many run, fewer only where a range would be empty: split_plan; the INT32 partials are exact, so
+    every choice gives the same bits).  With a schedule the ranges run on its 256-row tiles, without
+    one on the best tile for that number.  A forced schedule with `splits` None runs unsplit: the
+    launch timed is the one named.  None keeps the library's own plan.  These are the knobs the
+    harness tuner searches; both settings are thread-local."""
     if schedule is not None and schedule not in SCHEDULES:
         raise ValueError(f"unknown GEMM schedule {schedule!r}")
     if splits is not None and (isinstance(splits, bool) or not isinstance(splits, int) or not 1 <= splits <= 64):
@@ -222,7 +223,29 @@ def _cu_count(device):
     return _cu_count_of(device.index if device.index is not None else torch.cuda.current_device())
 
 
-TILES = ("256", "128", "64", "64-deep", "decode")
+TILES = ("256", "128", "64", "64-deep", "decode", "256x128")
+
+
+@contextlib.contextmanager
+def exact_splits():
+    """The library's split entry points run as many K ranges as a call names, for the calls this thread
+    makes inside the block (m5k_gemm_set_exact_splits)."""
+    lib, previous = _lib.load(), ctypes.c_int(0)
+    lib.m5k_gemm_set_exact_splits(1, ctypes.byref(previous))
+    try:
+        yield
+    finally:
+        lib.m5k_gemm_set_exact_splits(previous.value, None)
+
+
+def split_plan(mode, m, n, k, splits, cus=256):
+    """What the split entry point of mode "int8" or "fp8" launches for `splits` under this thread's
+    settings (m5k_gemm_split_plan; host only): (tile by name, K ranges that run; 1: unsplit)."""
+    tile, ranges = ctypes.c_int(0), ctypes.c_int(0)
+    lib = _lib.load()
+    if lib.m5k_gemm_split_plan(_PLAN_DTYPES[mode], m, n, k, cus, splits, ctypes.byref(tile), ctypes.byref(ranges)):
+        raise RuntimeError(lib.m5k_last_error().decode(errors="replace"))
+    return TILES[tile.value], ranges.value
 
 
 @functools.lru_cache(maxsize=4096)
@@ -442,12 +465,13 @@ def gemm(
             return c
         if splits > 1:
             workspace = torch.empty((splits, m, n), dtype=torch.int32, device=a.device)
-            _lib.call(
-                "m5k_gemm_i8_splitk",
-                _lib.ptr(a), _lib.ptr(b), m, n, k, _lib.ptr(a_scales), _lib.ptr(b_scales), _lib.ptr(c), out_code,
-                _lib.ptr(bias), _lib.ptr(bias_row_map), _lib.ptr(residual), _lib.ptr(gate), _lib.ptr(gate_row_map),
-                splits, _lib.ptr(workspace), workspace.numel(), stream,
-            )
+            with exact_splits() if forced_splits is not None else contextlib.nullcontext():
+                _lib.call(
+                    "m5k_gemm_i8_splitk",
+                    _lib.ptr(a), _lib.ptr(b), m, n, k, _lib.ptr(a_scales), _lib.ptr(b_scales), _lib.ptr(c), out_code,
+                    _lib.ptr(bias), _lib.ptr(bias_row_map), _lib.ptr(residual), _lib.ptr(gate),
+                    _lib.ptr(gate_row_map), splits, _lib.ptr(workspace), workspace.numel(), stream,
+                )
             return c
         _lib.call(
             "m5k_gemm_i8",
