@@ -8,6 +8,8 @@ of the reference) and rel-L2 1e-3 of the float64 product for FP32 output.
 
 from __future__ import annotations
 
+import contextlib
+
 import numpy as np
 import pytest
 import torch
@@ -278,7 +280,7 @@ def test_mxint8_gemm(shape, device):
 
 def _gemm_i8_call(entry, a, b, sa, sb, out, *, splits=None, bias=None, bias_map=None, residual=None, gate=None,
                   gate_map=None):
-    from m5kernels_amd import _lib
+    from m5kernels_amd import _lib, hip
 
     m, k = a.shape
     n = b.shape[0]
@@ -288,7 +290,10 @@ def _gemm_i8_call(entry, a, b, sa, sb, out, *, splits=None, bias=None, bias_map=
     if entry == "m5k_gemm_i8_splitk":
         ws = torch.full((splits, m, n), 12345, dtype=torch.int32, device=a.device)  # stale contents must not leak
         args += [splits, _lib.ptr(ws), ws.numel()]
-    _lib.call(entry, *args, _lib.stream_of(a))
+    with hip.exact_splits():  # the count that the caller names, not up to as many
+        if splits is not None:
+            assert hip.split_plan("int8", m, n, k, splits)[1] > 1
+        _lib.call(entry, *args, _lib.stream_of(a))
     return c
 
 
@@ -298,8 +303,8 @@ def _gemm_i8_call(entry, a, b, sa, sb, out, *, splits=None, bias=None, bias_map=
 @pytest.mark.parametrize("epilogue", ["bf16", "fp32", "fp16", "bias", "bias_table", "gate", "gate_table"])
 def test_splitk_bit_identical_to_plain(shape, splits, epilogue, device):
     """Split-K sums exact INT32 partials and applies the plain epilogue, so every output bit
-    matches m5k_gemm_i8 (K 2000 ends in a partial 64-byte slab; 16 splits of short K leave
-    some ranges shorter than a stage)."""
+    matches m5k_gemm_i8 (K 2000 ends in a partial stage; of 16 ranges of a short K fewer run, one
+    stage each)."""
     m, n, k = shape
     g = torch.Generator(device="cpu").manual_seed(m + n + k + splits)
     a = torch.randint(-127, 128, (m, k), generator=g, dtype=torch.int8).to(device)
@@ -322,15 +327,17 @@ def test_splitk_bit_identical_to_plain(shape, splits, epilogue, device):
 
 
 def test_splitk_plan_and_routing(device):
-    """gemm() takes the split path for few-tile shapes and the plain one otherwise; both are
-    bit-exact against the oracle's W8A8 epilogue."""
-    from m5kernels_amd.hip import splitk_plan
+    """gemm() hands few-tile shapes to the split entry point, which runs K ranges (128 x 1536 x 5376) or
+    an unsplit small tile (16 x 4096 x 4096), and the others to the plain one; bit-exact against the
+    oracle's W8A8 epilogue."""
+    from m5kernels_amd.hip import split_plan, splitk_plan
 
     assert splitk_plan(4096, 4096, 16384) == 1
     assert splitk_plan(128, 7168, 5376) > 1 and splitk_plan(16, 4096, 4096) > 1
     g = torch.Generator(device="cpu").manual_seed(3)
     for m, n, k in ((128, 1536, 5376), (16, 4096, 4096)):
         assert splitk_plan(m, n, k) > 1
+        assert (split_plan("int8", m, n, k, splitk_plan(m, n, k))[1] > 1) == (n == 1536)
         a = torch.randint(-127, 128, (m, k), generator=g, dtype=torch.int8).to(device)
         b = torch.randint(-127, 128, (n, k), generator=g, dtype=torch.int8).to(device)
         sa = (torch.rand(m, generator=g) + 0.5).to(device)
@@ -344,18 +351,19 @@ def test_splitk_plan_and_routing(device):
 
 # Shapes of 8+ rounds with a partial last round that gemm() splits by rows (256 CUs; the
 # library's mixed launch declines them, one shorter round saving under 5%): 2072 tiles (tail
-# rows 256, 5 K ranges), 2064 tiles (tail rows 256, 6 ranges), 2080 tiles with a ragged last
-# tile row (tail rows 332, 5 ranges).
+# rows 256, up to 5 K ranges), 2064 tiles (tail rows 256, up to 6 ranges), 2080 tiles with a ragged
+# last tile row (tail rows 332, up to 5 ranges).
 _TAIL_CASES = [(18944, 7168, 4096), (33024, 4096, 4096), (33100, 4096, 4096)]
 
 
 @pytest.mark.parametrize("shape", _TAIL_CASES)
 @pytest.mark.parametrize("epilogue", ["bf16", "fp32", "fp16", "bias", "bias_table", "gate", "gate_table"])
 def test_tail_split_bit_identical_to_plain(shape, epilogue, device):
-    """gemm() runs whole tile rows as a plain launch and the rest as split-K, slicing every
-    row-indexed operand (scales, row maps, residual, output) at the same row; the result
-    matches one plain m5k_gemm_i8 launch bit for bit."""
-    from m5kernels_amd.hip import launch_plan, tail_split_plan
+    """gemm() runs whole tile rows as a plain launch and the rest through the split entry point, slicing
+    every row-indexed operand (scales, row maps, residual, output) at the same row; the result
+    matches one plain m5k_gemm_i8 launch bit for bit, with the library's choice for the rest (an
+    unsplit small tile here) and with the K ranges that the plan names."""
+    from m5kernels_amd.hip import exact_splits, launch_plan, tail_split_plan
 
     m, n, k = shape
     cus = torch.cuda.get_device_properties(0).multi_processor_count
@@ -382,6 +390,9 @@ def test_tail_split_bit_identical_to_plain(shape, epilogue, device):
     plain = _gemm_i8_call("m5k_gemm_i8", a, b, sa, sb, out, **kw)
     y = gemm(a, b, "int8", a_scales=sa, b_scales=sb, output_dtype=out, **call_kw)
     view = torch.int16 if out != torch.float32 else torch.int32
+    assert torch.equal(plain.view(view), y.view(view))
+    with exact_splits():
+        y = gemm(a, b, "int8", a_scales=sa, b_scales=sb, output_dtype=out, **call_kw)
     assert torch.equal(plain.view(view), y.view(view))
 
 
@@ -562,9 +573,9 @@ def test_ops_launch_on_the_current_stream(device):
 
 @pytest.mark.parametrize("shape", [(128, 5376, 14336), (16, 4096, 4096), (300, 1000, 1024), (1, 96, 5376)])
 def test_fp8_split_k_against_float64_and_unsplit(shape, device):
-    """Short-M FP8 GEMMs take the split-K launch (FP32 partials summed in split order): within the
-    FP8 bar of the decoded float64 product, within FP32 rounding of the unsplit launch, and the
-    same bits on a second call."""
+    """Short-M FP8 GEMMs in as many K ranges as gemm() plans at most (FP32 partials summed in split
+    order): within the FP8 bar of the decoded float64 product, within FP32 rounding of the unsplit
+    launch, and the same bits on a second call.  Then the same for the library's own choice."""
     from m5kernels_amd import hip
 
     m, n, k = shape
@@ -577,11 +588,16 @@ def test_fp8_split_k_against_float64_and_unsplit(shape, device):
     bq, sb = quantize(b, "fp8")
     decoded = (ref.dequantize(np_of(aq), np_of(sa), "fp8").astype(np.float64)
                @ ref.dequantize(np_of(bq), np_of(sb), "fp8").astype(np.float64).T)
-    y_split = gemm(aq, bq, "fp8", a_scales=sa, b_scales=sb)
     with hip.launch_override("plain"):
         y_plain = gemm(aq, bq, "fp8", a_scales=sa, b_scales=sb)
-    assert ref.metrics(np_of(y_split), decoded)["relative_l2"] < 1e-4
-    assert ref.metrics(np_of(y_split), np_of(y_plain).astype(np.float64))["relative_l2"] < 1e-5
-    assert torch.equal(gemm(aq, bq, "fp8", a_scales=sa, b_scales=sb), y_split)
-    y16 = gemm(aq, bq, "fp8", a_scales=sa, b_scales=sb, output_dtype=torch.bfloat16)
-    assert ref.metrics(y16.float().cpu().numpy(), decoded)["relative_l2"] < 0.008
+    for setting in (hip.exact_splits(), contextlib.nullcontext()):
+        with setting:
+            planned = hip.splitk_plan(m, n, k, 256, skinny=False)
+            ranges = hip.split_plan("fp8", m, n, k, planned)[1]
+            assert ranges > 1 or isinstance(setting, contextlib.nullcontext)
+            y_split = gemm(aq, bq, "fp8", a_scales=sa, b_scales=sb)
+            assert ref.metrics(np_of(y_split), decoded)["relative_l2"] < 1e-4
+            assert ref.metrics(np_of(y_split), np_of(y_plain).astype(np.float64))["relative_l2"] < 1e-5
+            assert torch.equal(gemm(aq, bq, "fp8", a_scales=sa, b_scales=sb), y_split)
+            y16 = gemm(aq, bq, "fp8", a_scales=sa, b_scales=sb, output_dtype=torch.bfloat16)
+            assert ref.metrics(y16.float().cpu().numpy(), decoded)["relative_l2"] < 0.008

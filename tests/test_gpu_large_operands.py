@@ -39,9 +39,9 @@ def test_int8_a_operand_over_2gib(device):
 
 
 def test_int8_weight_over_2gib_split_k_routing(device):
-    """Short M with a 2 GiB weight: gemm() plans split-K (n * k >= 2^31), which the library
-    accepts now that each workgroup addresses a 256-row window."""
-    from m5kernels_amd.hip import splitk_plan
+    """Short M with a 2 GiB weight (n * k >= 2^31): gemm() goes to the split entry point, whose workgroups
+    each address their own rows only; the library's choice, then the K ranges that the plan names."""
+    from m5kernels_amd.hip import exact_splits, split_plan, splitk_plan
 
     m, n, k = 16, 16_384, 131_072  # W is 2 GiB
     assert n * k >= 2**31 and splitk_plan(m, n, k) > 1
@@ -54,6 +54,9 @@ def test_int8_weight_over_2gib_split_k_routing(device):
     cols = _far_rows(n)
     expected = ref.c_i8_epilogue(ref.c_gemm_i8_acc(np_of(a), np_of(b[cols])), np_of(sa), np_of(sb[cols]))
     np.testing.assert_array_equal(bits_of(y[:, cols]), expected)
+    with exact_splits():
+        assert split_plan("int8", m, n, k, splitk_plan(m, n, k))[1] > 1
+        assert torch.equal(gemm(a, b, "int8", a_scales=sa, b_scales=sb, output_dtype=torch.bfloat16), y)
     del b
 
 

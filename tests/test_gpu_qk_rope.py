@@ -255,13 +255,15 @@ def test_grouped_qkv_equals_staged(mode, rope_half, m, heads, device):
 
 @pytest.mark.parametrize("m", [1, 17, 128, 200])
 def test_short_m_routing_matches_fused_kernel(m, device):
-    """Short-M INT8 projections take the split-K GEMM plus the staged postprocess; the result
-    equals the fused kernel's (called through the C ABI directly) bit for bit."""
+    """Short-M INT8 projections take the plain GEMM (the decode tile at 1 and 17 rows, K ranges of 64 x 64
+    tiles at 128 and 200) plus the staged postprocess; the result equals the fused kernel's (called
+    through the C ABI directly) bit for bit."""
     from m5kernels_amd import _lib
-    from m5kernels_amd.hip import splitk_plan
+    from m5kernels_amd.hip import split_plan, splitk_plan
 
     n, k = 768, 5376
     assert splitk_plan(m, n, k) > 1
+    assert (split_plan("int8", m, n, k, splitk_plan(m, n, k))[1] > 1) == (m > 32)
     rng = np.random.default_rng(m)
     a, sa = quantize(torch.from_numpy(rng.standard_normal((m, k), dtype=np.float32)).to(device), "int8")
     b, sb = quantize(torch.from_numpy(rng.standard_normal((n, k), dtype=np.float32)).to(device), "int8")

@@ -10,9 +10,17 @@ from __future__ import annotations
 import pytest
 import torch
 
-from m5kernels_amd import _lib
+from m5kernels_amd import _lib, hip
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(autouse=True)
+def named_counts_run():
+    """Every call here runs the K ranges that it names, so that the scratch array is used."""
+    with hip.exact_splits():
+        yield
+
 
 SCRATCH_ELEMS = 16 * 1024 * 1024  # M5K_SCRATCH_ELEMS in include/m5k.h
 
@@ -54,11 +62,14 @@ def test_noalloc_matches_workspace_form_twice(epilogue, out_dtype, device):
     # A large call, then a smaller one: the second must not see the first one's partials.
     for (m, n, k, splits), seed in (((256, 4096, 4096, 8), 1), ((128, 1536, 5376, 3), 2)):
         assert splits * m * n <= SCRATCH_ELEMS
+        assert hip.split_plan("int8", m, n, k, splits)[1] == splits
         a, b, sa, sb, extra = _operands(m, n, k, seed, device, epilogue)
         got = _call("m5k_gemm_i8_splitk_noalloc", a, b, sa, sb, extra, splits, out_dtype)
         want = _call("m5k_gemm_i8_splitk", a, b, sa, sb, extra, splits, out_dtype)
         torch.cuda.synchronize()
         assert torch.equal(got.view(view), want.view(view)), (m, n, k, splits)
+        unsplit = _call("m5k_gemm_i8_splitk", a, b, sa, sb, extra, 1, out_dtype)
+        assert torch.equal(got.view(view), unsplit.view(view)), (m, n, k, splits)
 
 
 def test_noalloc_rejects_sizes_beyond_the_scratch_array(device):
@@ -86,6 +97,7 @@ def test_noalloc_replays_under_graph_capture(device):
     with torch.cuda.graph(graph, stream=side):
         _lib.call("m5k_gemm_i8_splitk_noalloc", *args, _lib.stream_of(a))
     other = _operands(256, 2048, 1024, 5, device, "plain")
+    assert hip.split_plan("int8", m, n, k, splits)[1] == 3 and hip.split_plan("int8", 256, 2048, 1024, 4)[1] == 4
     for _ in range(3):
         c.fill_(float("nan"))
         _call("m5k_gemm_i8_splitk_noalloc", *other, 4, torch.bfloat16)  # eager use of the scratch between replays
