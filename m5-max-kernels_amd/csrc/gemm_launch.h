@@ -241,7 +241,8 @@ inline plan::Choice plan_tile(int mode, int64_t m, int64_t n, int64_t kb, int cu
     int64_t full = -1;
     if (forced_schedule(md16, mode == I8, m, n, cus, full) >= 0) return none;
     if (mode != I8 && kb < 8 * BKB) return none;
-    limit_us = std::min(limit_us, plan::tile256_us(units_256(md16, m, n, cus), n, kb));
+    const double units = units_256(md16, m, n, cus);
+    limit_us = std::min(limit_us, max_splits > 1 ? plan::tile256_us(units, n, kb) : plan::unsplit256_us(units, n, kb));
   }
   return plan::choose(m, n, kb, cus, aligned, max_splits, limit_us);
 }

@@ -14,8 +14,12 @@
 //   256-row schedules  u rounds' worth of tiles: u (13 + 10)         4096 x 4096 x 4096 INT8 54.5 us
 //
 // Every product streams its weight once, at about 5.2 TB/s at best; the 256-row tiles, with one stage
-// ahead, at about 2 TB/s where the Infinity Cache does not hold it (402 x 14336 x 16384: 152 us).  A
-// split over K adds a second launch and its 4-byte partial sums, written and read at about 6 TB/s.
+// ahead, at about 2 TB/s where the Infinity Cache does not hold it (402 x 14336 x 16384: 152 us), and
+// at 3 TB/s where it does: the other tiles' rates are of weights that it holds, too.  With 2 TB/s for
+// both, two rounds of 128 x 128 tiles were taken for one round of 256 x 128 halves (BF16 256 x 21504 x
+// 4096: 70.0 us against 55.5 with one weight, 83.0 against 76.0 with weights in turn; INT8 256 x 21504 x
+// 5376: 49.8 against 39.9, 59.3 against 57.8).  K ranges are weighed against the 2 TB/s.  A split
+// over K adds a second launch and its 4-byte partial sums, written and read at about 6 TB/s.
 #pragma once
 
 #include <stdint.h>
@@ -76,8 +80,15 @@ inline double tile_us(int tile, int64_t m, int64_t n, int64_t kb, int cus, int s
 }
 
 // `units_256`: the 256-row schedules' time in 256 x 256 tile times; they stream the weight at 2 MB/us.
-inline double tile256_us(double units_256, int64_t n, int64_t kb) {
-  return with_stream(units_256 * (13.0 + 10.0e-3 * static_cast<double>(kb)), n, kb, 2.0e6);
+inline double tile256_us(double units_256, int64_t n, int64_t kb, double bytes_per_us = 2.0e6) {
+  return with_stream(units_256 * (13.0 + 10.0e-3 * static_cast<double>(kb)), n, kb, bytes_per_us);
+}
+
+// The same beside other unsplit tiles: 3 MB/us for a weight that the Infinity Cache holds.
+inline double unsplit256_us(double units_256, int64_t n, int64_t kb) {
+  constexpr double kInfinityCache = 256.0e6;
+  const double weight = static_cast<double>(n) * static_cast<double>(kb);
+  return tile256_us(units_256, n, kb, weight <= kInfinityCache ? 3.0e6 : 2.0e6);
 }
 
 // The fastest tile of an [m, n] output with rows of kb bytes and min_splits to max_splits K ranges, or

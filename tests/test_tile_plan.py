@@ -59,3 +59,15 @@ def test_a_long_k_splits_where_decode_would_leave_cus_idle():
     # 30 x 2048 x 16384: 128 decode workgroups of 32 rows took 24 us, K ranges of ring tiles 14 us.
     assert hip._tile_plan.__wrapped__("int8", 30, 2048, 16384, 256, True, None, 16) != "decode"
     assert hip._tile_plan.__wrapped__("int8", 1, 4096, 4096, 256, True, None, 4) == "decode"
+
+
+def test_one_round_of_half_tiles_is_not_given_up_for_two_rounds_of_small_ones():
+    # 84 tiles of 256 x 256, as 168 halves in one round: BF16 256 x 21504 x 4096 55.5 us against 70.0 us on
+    # 336 tiles of 128 x 128, INT8 256 x 21504 x 5376 39.9 us against 49.8 us.
+    for m in (200, 256):
+        assert _plan("bf16", m, 21504, 4096) == "256" and _plan("bf16", m, 21504, 5376) == "256"
+        assert _plan("int8", m, 21504, 5376) == "256" and _plan("fp8", m, 21504, 5376) == "256"
+    # One round of small tiles stays ahead (BF16 128 x 21504 x 4096: 36.8 us against 50.4 us), and two rounds where
+    # the weight is larger than the Infinity Cache (BF16 400 x 16384 x 14336: 253.7 us against 285.2 us).
+    assert _plan("bf16", 128, 21504, 4096) == "128" and _plan("int8", 128, 21504, 5376) == "128"
+    assert _plan("bf16", 400, 16384, 14336) == "128"
