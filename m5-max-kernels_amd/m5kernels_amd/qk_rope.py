@@ -22,14 +22,17 @@ from .hip import gemm, splitk_plan, tile_plan
 HEAD_DIM = 128
 
 
-def _staged(a, b, mode):
+def _staged(a, b, mode, grouped=False):
     """Whether the projection runs as the plain GEMM and the staged postprocess: where the GEMM's best
     tile is smaller than a head (few rows: 128 x 7168 x 5376 INT8 14 us + 4 us against 26 us fused on
-    one-head tiles), or a split over K.  The fused kernel's tiles otherwise: it takes the plain GEMM's
-    choice between one-head and 256-row tiles.  Both give the same bits."""
+    one-head tiles), or where gemm() may split K over 256-row tiles.  The fused kernel's tiles otherwise:
+    it takes the plain GEMM's choice between one-head and 256-row tiles.  Both give the plain GEMM's bits
+    through the postprocess.  The grouped layout (Q/K/V) is wide, so 256-row tiles hold their round and
+    K ranges with a second and a third pass over the output cost more than they save: 768 x 10752 x 1024
+    INT8 16.3 us fused against 27.3 us, 256 x 21504 x 1024 15.8 us against 22.0 us."""
     tile = tile_plan(mode, a, b)
     if tile == "256":
-        return mode == "int8" and splitk_plan(a.shape[0], b.shape[0], a.shape[1]) > 1
+        return not grouped and mode == "int8" and splitk_plan(a.shape[0], b.shape[0], a.shape[1]) > 1
     return tile != "128"
 
 
@@ -193,7 +196,7 @@ def projection_qkv_rope(a, w, q_gamma, k_gamma, cos, sin, mode="int8", *, a_scal
     w = _lib.device_tensor(w, "w")
     q_gamma, cos, sin = _tables(q_gamma, cos, sin)
     k_gamma = _lib.aligned_device_tensor(k_gamma, "k_gamma")
-    staged = _staged(a, w, mode)
+    staged = _staged(a, w, mode, grouped=True)
     if staged:
         projected = gemm(a, w, mode, a_scales=a_scales, b_scales=w_scales, output_dtype=torch.bfloat16)
     q, kk, v = (torch.empty((heads, m, HEAD_DIM), dtype=torch.bfloat16, device=a.device) for _ in range(3))
