@@ -1,5 +1,6 @@
-// Native front of the two calls that every quantized linear makes, quantize() and gemm(): the
-// argument checks, the output allocation and the launch of a plain call, without the interpreter.
+// Native front of the calls that a projection makes, quantize(), gemm() and the Q/K and Q/K/V
+// projections: the argument checks, the output allocation and the launches of a plain call, without the
+// interpreter.
 //
 // Each function takes a call only if it can see that the Python front (hip.py) would accept it and
 // launch at once: plain CUDA tensors, contiguous, of the right dtypes and shapes, no forced schedule.
@@ -7,13 +8,15 @@
 // is decided here.  The launches are the same C ABI calls, with the interpreter lock released.
 //
 // Measured on a [1, 256] activation: quantize 7.3 -> 4.6 us of host time, gemm 9.4 -> 4.4 us, of which
-// the HIP launch takes about 3 each.
+// the HIP launch takes about 3 each.  The projections' staged form, two launches, takes
+// 18 to 20 us through Python and 8 to 10 us here; the fused one 10 to 13 and 5 to 6 us.
 #include <Python.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/extension.h>
 
+#include <cmath>
 #include <mutex>
 #include <unordered_map>
 
@@ -23,6 +26,9 @@ namespace {
 
 PyObject* g_stream_of = nullptr;  // torch's raw stream handle of a device index
 PyObject* g_splits = nullptr;     // hip._native_splits(mode, m, n, k, device index) -> K ranges, 0: not here
+PyObject* g_staged = nullptr;     // hip._native_staged(mode, m, n, k, device index, aligned, grouped) -> 0 or 1
+
+enum Mode { INT8, FP8, B16, H16 };
 
 int dtype_code(at::ScalarType t) {
   switch (t) {
@@ -104,19 +110,20 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// K ranges of an aligned INT8 or FP8 product, from hip.py's planner, kept per shape and settings of
-// the environment (bounded: emptied when full).
+// What hip.py's planner says of a shape, kept per shape and settings of the environment (bounded:
+// emptied when full).  `what`: the mode, and for a projection's route bits 4 (a route), 5 (aligned
+// operands) and 6 (grouped layout).
 struct Key {
-  int mode, device, state;
+  int what, device, state;
   int64_t m, n, k;
   bool operator==(const Key& o) const {
-    return mode == o.mode && device == o.device && state == o.state && m == o.m && n == o.n && k == o.k;
+    return what == o.what && device == o.device && state == o.state && m == o.m && n == o.n && k == o.k;
   }
 };
 struct Hash {
   size_t operator()(const Key& x) const {
     uint64_t h = 1469598103934665603ull;
-    for (uint64_t v : {uint64_t(x.mode), uint64_t(x.device), uint64_t(x.state), uint64_t(x.m), uint64_t(x.n), uint64_t(x.k)})
+    for (uint64_t v : {uint64_t(x.what), uint64_t(x.device), uint64_t(x.state), uint64_t(x.m), uint64_t(x.n), uint64_t(x.k)})
       h = (h ^ v) * 1099511628211ull, h ^= h >> 29;
     return h;
   }
@@ -124,14 +131,14 @@ struct Hash {
 std::mutex g_mutex;
 std::unordered_map<Key, int, Hash> g_plans;
 
-int planned_splits(const Key& key, PyObject* mode) {  // -1: a Python error is set
+template <class Ask>
+int planned(const Key& key, Ask ask) {  // -1: a Python error is set
   {
     std::lock_guard<std::mutex> lock(g_mutex);
     const auto it = g_plans.find(key);
     if (it != g_plans.end()) return it->second;
   }
-  PyObject* r = PyObject_CallFunction(g_splits, "OLLLi", mode, (long long)key.m, (long long)key.n, (long long)key.k,
-                                      key.device);
+  PyObject* r = ask();
   if (!r) return -1;
   const long v = PyLong_AsLong(r);
   Py_DECREF(r);
@@ -142,11 +149,27 @@ int planned_splits(const Key& key, PyObject* mode) {  // -1: a Python error is s
   return static_cast<int>(v);
 }
 
+// K ranges of an aligned INT8 or FP8 product.
+int planned_splits(const Key& key, PyObject* mode) {
+  return planned(key, [&] {
+    return PyObject_CallFunction(g_splits, "OLLLi", mode, (long long)key.m, (long long)key.n, (long long)key.k, key.device);
+  });
+}
+
+// Whether a projection runs as the GEMM and a postprocess.
+int planned_staged(const Key& key, PyObject* mode, bool aligned, bool grouped) {
+  return planned(key, [&] {
+    return PyObject_CallFunction(g_staged, "OLLLiii", mode, (long long)key.m, (long long)key.n, (long long)key.k,
+                                 key.device, int(aligned), int(grouped));
+  });
+}
+
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
 // gemm(a, b, mode, a_scales, b_scales, output_dtype, bias, bias_row_map, residual, gate, gate_row_map).
 PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   HANDLE_TH_ERRORS
   if (nargs != 11 || !PyUnicode_Check(args[2])) Py_RETURN_NONE;
-  enum { INT8, FP8, B16, H16 };
   PyObject* mo = args[2];
   const int mode = PyUnicode_CompareWithASCIIString(mo, "int8") == 0   ? INT8
                    : PyUnicode_CompareWithASCIIString(mo, "bf16") == 0 ? B16
@@ -212,7 +235,7 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (state & 0xF) Py_RETURN_NONE;  // a schedule is forced
   const void *ap = a->data_ptr(), *bp = b->data_ptr();
   int splits = 1;
-  if (quant && k % 16 == 0 && ((reinterpret_cast<uintptr_t>(ap) | reinterpret_cast<uintptr_t>(bp)) & 15u) == 0) {
+  if (quant && k % 16 == 0 && aligned16(ap) && aligned16(bp)) {
     splits = planned_splits(Key{mode, dev.index(), state, m, n, k}, mo);
     if (splits < 0) return nullptr;
     if (splits == 0) Py_RETURN_NONE;
@@ -255,22 +278,151 @@ PyObject* gemm(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind(stream_of, splits): the Python callables above.
+// The Q/K projection (args: a, b, gamma, cos, sin, mode, a_scales, b_scales, epsilon) and the grouped
+// Q/K/V one (a, w, q_gamma, k_gamma, cos, sin, mode, a_scales, w_scales, epsilon), by the route that
+// hip.projection_staged names.
+constexpr int64_t HEAD = 128;
+
+PyObject* project(PyObject* const* args, bool grouped) {
+  const int at = grouped ? 4 : 3;  // index of cos
+  PyObject* mo = args[at + 2];
+  if (!PyUnicode_Check(mo)) Py_RETURN_NONE;
+  const bool i8 = PyUnicode_CompareWithASCIIString(mo, "int8") == 0;
+  if (!i8 && PyUnicode_CompareWithASCIIString(mo, "bf16") != 0) Py_RETURN_NONE;
+  const at::Tensor *a = plain(args[0]), *b = plain(args[1]);
+  const at::ScalarType operand = i8 ? at::kChar : at::kBFloat16;
+  if (!a || !b || a->dim() != 2 || b->dim() != 2 || a->scalar_type() != operand || b->scalar_type() != operand ||
+      a->device() != b->device())
+    Py_RETURN_NONE;
+  const c10::Device dev = a->device();
+  const int64_t m = a->size(0), k = a->size(1), n = b->size(0), block = grouped ? 3 * HEAD : HEAD;
+  if (b->size(1) != k || m == 0 || n == 0 || k == 0 || n % block || (i8 && k > 131071)) Py_RETURN_NONE;
+  const float *sa = nullptr, *sb = nullptr;
+  if (i8) {
+    const at::Tensor *ta = plain(args[at + 3]), *tb = plain(args[at + 4]);
+    if (!vector_of(ta, m, at::kFloat, dev) || !vector_of(tb, n, at::kFloat, dev)) Py_RETURN_NONE;
+    sa = static_cast<const float*>(ta->data_ptr());
+    sb = static_cast<const float*>(tb->data_ptr());
+  } else if (args[at + 3] != Py_None || args[at + 4] != Py_None) {
+    Py_RETURN_NONE;
+  }
+  const at::Tensor *g = plain(args[2]), *gk = grouped ? plain(args[3]) : g, *cos = plain(args[at]), *sin = plain(args[at + 1]);
+  if (!vector_of(g, HEAD, at::kBFloat16, dev) || !vector_of(gk, HEAD, at::kBFloat16, dev) || !aligned16(g->data_ptr()) ||
+      !aligned16(gk->data_ptr()))
+    Py_RETURN_NONE;
+  for (const at::Tensor* t : {cos, sin})
+    if (!t || t->dim() != 2 || t->size(0) != m || t->scalar_type() != at::kBFloat16 || t->device() != dev) Py_RETURN_NONE;
+  const int64_t half = cos->size(1);
+  if (half < 1 || half > HEAD / 2 || sin->size(1) != half) Py_RETURN_NONE;
+  if (!PyFloat_CheckExact(args[at + 5])) Py_RETURN_NONE;
+  const float eps = static_cast<float>(PyFloat_AS_DOUBLE(args[at + 5]));
+  if (!(eps > 0.0f) || !std::isfinite(eps)) Py_RETURN_NONE;
+  const int state = m5k_gemm_schedule_state();
+  if (state & 0xF) Py_RETURN_NONE;  // a schedule is forced
+  const void *ap = a->data_ptr(), *bp = b->data_ptr();
+  const int64_t row = k * (i8 ? 1 : 2);
+  const bool whole = row % 16 == 0 && aligned16(ap) && aligned16(bp), aligned = whole && row <= int64_t(1) << 23;
+  const int mode = i8 ? INT8 : B16;
+  const int staged = planned_staged(Key{mode | 16 | (aligned ? 32 : 0) | (grouped ? 64 : 0), dev.index(), state, m, n, k},
+                                    mo, aligned, grouped);
+  if (staged < 0) return nullptr;
+  int splits = 1;
+  if (staged && i8 && whole) {
+    splits = planned_splits(Key{mode, dev.index(), state, m, n, k}, mo);
+    if (splits < 0) return nullptr;
+    if (splits == 0) Py_RETURN_NONE;
+  }
+  void* stream = nullptr;
+  if (!stream_of(dev, &stream)) return nullptr;
+  const int64_t heads = n / block;
+  at::Tensor y[3], projected, workspace;
+  for (int i = 0; i < (grouped ? 3 : 1); ++i) y[i] = empty({heads, m, HEAD}, at::kBFloat16, dev);
+  if (staged) projected = empty({m, n}, at::kBFloat16, dev);
+  if (splits > 1) workspace = empty({splits, m, n}, at::kInt, dev);
+  void* yp[3] = {y[0].data_ptr(), grouped ? y[1].data_ptr() : nullptr, grouped ? y[2].data_ptr() : nullptr};
+  void* pp = staged ? projected.data_ptr() : nullptr;
+  auto* wp = splits > 1 ? static_cast<int32_t*>(workspace.data_ptr()) : nullptr;
+  const void *gp = g->data_ptr(), *gkp = gk->data_ptr(), *cp = cos->data_ptr(), *sp = sin->data_ptr();
+  auto* ai = static_cast<const int8_t*>(ap);
+  auto* bi = static_cast<const int8_t*>(bp);
+  const int r = static_cast<int>(half), dtype = i8 ? M5K_I8 : M5K_BF16;
+  const char* name = nullptr;
+  int rc = 0;
+  Py_BEGIN_ALLOW_THREADS
+  if (staged) {
+    if (splits > 1) {
+      name = "m5k_gemm_i8_splitk";
+      rc = m5k_gemm_i8_splitk(ai, bi, m, n, k, sa, sb, pp, M5K_BF16, nullptr, nullptr, nullptr, nullptr, nullptr, splits,
+                              wp, splits * m * n, stream);
+    } else if (i8) {
+      name = "m5k_gemm_i8";
+      rc = m5k_gemm_i8(ai, bi, m, n, k, sa, sb, pp, M5K_BF16, nullptr, nullptr, nullptr, nullptr, nullptr, stream);
+    } else {
+      name = "m5k_gemm_float";
+      rc = m5k_gemm_float(ap, bp, M5K_BF16, m, n, k, pp, M5K_BF16, nullptr, nullptr, nullptr, stream);
+    }
+    if (rc == 0 && grouped) {
+      name = "m5k_qkv_norm_rope";
+      rc = m5k_qkv_norm_rope(pp, m, heads, gp, gkp, cp, sp, r, eps, yp[0], yp[1], yp[2], stream);
+    } else if (rc == 0) {
+      name = "m5k_qk_norm_rope";
+      rc = m5k_qk_norm_rope(pp, m, n, gp, cp, sp, r, eps, yp[0], stream);
+    }
+  } else if (grouped) {
+    name = "m5k_projection_qkv_rope";
+    rc = m5k_projection_qkv_rope(ap, bp, dtype, m, heads, k, sa, sb, gp, gkp, cp, sp, r, eps, yp[0], yp[1], yp[2], stream);
+  } else {
+    name = "m5k_projection_qk_rope";
+    rc = m5k_projection_qk_rope(ap, bp, dtype, m, n, k, sa, sb, gp, cp, sp, r, eps, yp[0], stream);
+  }
+  Py_END_ALLOW_THREADS
+  if (rc) return failed(name, rc);
+  if (!grouped) return THPVariable_Wrap(std::move(y[0]));
+  PyObject* out = PyTuple_New(3);
+  for (int i = 0; out && i < 3; ++i) {
+    PyObject* o = THPVariable_Wrap(std::move(y[i]));
+    if (!o) {
+      Py_CLEAR(out);
+      break;
+    }
+    PyTuple_SET_ITEM(out, i, o);
+  }
+  return out;
+}
+
+PyObject* qk(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 9) Py_RETURN_NONE;
+  return project(args, false);
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* qkv(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  HANDLE_TH_ERRORS
+  if (nargs != 10) Py_RETURN_NONE;
+  return project(args, true);
+  END_HANDLE_TH_ERRORS
+}
+
+// bind(stream_of, splits, staged): the Python callables above.
 PyObject* bind(PyObject*, PyObject* args) {
-  PyObject *s, *p;
-  if (!PyArg_ParseTuple(args, "OO", &s, &p)) return nullptr;
-  Py_INCREF(s);
-  Py_INCREF(p);
-  Py_XDECREF(g_stream_of);
-  Py_XDECREF(g_splits);
-  g_stream_of = s;
-  g_splits = p;
+  PyObject *s, *p, *q;
+  if (!PyArg_ParseTuple(args, "OOO", &s, &p, &q)) return nullptr;
+  PyObject** slots[] = {&g_stream_of, &g_splits, &g_staged};
+  PyObject* given[] = {s, p, q};
+  for (int i = 0; i < 3; ++i) {
+    Py_INCREF(given[i]);
+    Py_XDECREF(*slots[i]);
+    *slots[i] = given[i];
+  }
   Py_RETURN_NONE;
 }
 
 PyMethodDef methods[] = {
     {"quantize", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(quantize)), METH_FASTCALL, nullptr},
     {"gemm", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(gemm)), METH_FASTCALL, nullptr},
+    {"qk", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(qk)), METH_FASTCALL, nullptr},
+    {"qkv", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(qkv)), METH_FASTCALL, nullptr},
     {"bind", bind, METH_VARARGS, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 

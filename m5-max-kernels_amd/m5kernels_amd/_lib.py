@@ -107,7 +107,7 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
 
 
 def load_fast():
-    """The native front of quantize() and gemm() (binding/fast_ops.cpp), linked against libm5k.so, or
+    """The native front of quantize(), gemm() and the projections (binding/fast_ops.cpp), linked against libm5k.so, or
     None where the libraries have not been built.  One that does not load, or that was compiled for
     another C ABI or another torch (left from an older build), warns: the same kernels then run with
     the checks in Python."""

@@ -3,7 +3,7 @@
 Every translation unit under ``csrc/`` is compiled to an object under ``_build/``
 (in parallel), then linked into ``lib/libm5k.so`` next to this package.  The measurement
 kernels under ``diag/`` (bench.py's MFMA ceiling) go into ``lib/libm5k_diag.so``, the native
-front of quantize() and gemm() under ``binding/`` (host code, against torch's headers) into
+front of the linears and projections under ``binding/`` (host code, against torch's headers) into
 ``lib/m5k_fast.so``; where those headers are missing the other two are built all the same.
 Flags:
 
@@ -118,8 +118,8 @@ def _front_includes() -> list[str]:
 
 
 def _compile_fast(force: bool) -> Path | None:
-    """The native front of quantize() and gemm(): host code against torch's headers (None without
-    them: quantize() and gemm() then run their checks in Python)."""
+    """The native front of the linears and projections: host code against torch's headers (None without
+    them: the checks then run in Python)."""
     import torch
 
     includes = _front_includes()

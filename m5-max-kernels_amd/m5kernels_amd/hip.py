@@ -50,8 +50,9 @@ def quantize(x, mode, tag="packed"):
     scale, returned as uint8 exponent bytes [rows, K/32] (e + 127, numerics.py:33-41).
     Mirrors metal.quantize (metal.py:27-44).
     """
-    if _fast is not None:
-        done = _fast.quantize(x, mode)
+    fast = _fast
+    if fast is not None:
+        done = fast.quantize(x, mode)
         if done is not None:
             return done
     rows, k = x.shape
@@ -304,6 +305,26 @@ def _native_splits(mode, m, n, k, index):
     return 0 if tail is not None else splits
 
 
+def projection_staged(tile, mode, m, n, k, grouped):
+    """Whether a Q/K (grouped: Q/K/V) projection whose plain GEMM would take `tile` runs as that GEMM and
+    the staged postprocess: where the tile is smaller than a head (few rows: 128 x 7168 x 5376 INT8 14 us +
+    4 us against 26 us fused on one-head tiles), or where gemm() may split K over 256-row tiles.  The
+    fused kernel's tiles otherwise: it takes the plain GEMM's choice between one-head and 256-row tiles.
+    Either way the bits are those of the plain GEMM through the postprocess.  The grouped layout is wide,
+    so 256-row tiles hold their round, and K ranges with a second and a third pass over the output cost
+    more than they save: 768 x 10752 x 1024 INT8 16.3 us fused against 27.3 us, 256 x 21504 x 1024 15.8 us
+    against 22.0 us."""
+    if tile == "256":
+        return not grouped and mode == "int8" and splitk_plan(m, n, k) > 1
+    return tile != "128"
+
+
+def _native_staged(mode, m, n, k, index, aligned, grouped):
+    """projection_staged for the native front, which keeps it per shape and m5k_gemm_schedule_state."""
+    tile = _tile_plan(mode, m, n, k, _cu_count_of(index), bool(aligned), (None, _environ_schedule()))
+    return int(projection_staged(tile, mode, m, n, k, bool(grouped)))
+
+
 @functools.lru_cache(maxsize=4096)
 def _f8_splits(m, n, k, cus, forced):
     """K ranges per tile of an aligned FP8 linear (1: the plain launch), cached per shape, CU
@@ -337,8 +358,9 @@ def gemm(
     [P,N] with gate_row_map[M]); that requires BF16 output and cannot be combined with
     a bias.  output_dtype defaults to float32.  Mirrors metal.gemm (metal.py:158-269).
     """
-    if _fast is not None and tile is _TILE and getattr(_override, "splits", None) is None:
-        c = _fast.gemm(a, b, mode, a_scales, b_scales, output_dtype, bias, bias_row_map, residual, gate, gate_row_map)
+    fast = _fast
+    if fast is not None and tile is _TILE and getattr(_override, "splits", None) is None:
+        c = fast.gemm(a, b, mode, a_scales, b_scales, output_dtype, bias, bias_row_map, residual, gate, gate_row_map)
         if c is not None:
             return c
     m, k = a.shape
@@ -602,7 +624,7 @@ class _NativeFront:
             if not self._done and _lib.LIB_PATH.exists():
                 self._module = _lib.load_fast()
                 if self._module is not None:
-                    self._module.bind(_lib._current_raw_stream, _native_splits)
+                    self._module.bind(_lib._current_raw_stream, _native_splits, _native_staged)
                 self._done = True
                 if _fast is self:
                     _fast = self._module
@@ -615,6 +637,14 @@ class _NativeFront:
     def gemm(self, *args):
         module = self._load()
         return None if module is None else module.gemm(*args)
+
+    def qk(self, *args):
+        module = self._load()
+        return None if module is None else module.qk(*args)
+
+    def qkv(self, *args):
+        module = self._load()
+        return None if module is None else module.qkv(*args)
 
 
 _fast = _NativeFront()

@@ -16,24 +16,16 @@ import struct
 
 import torch
 
-from . import _lib
-from .hip import gemm, splitk_plan, tile_plan
+from . import _lib, hip
+from .hip import gemm, tile_plan
 
 HEAD_DIM = 128
+_TILE = (32, 128, 4, 1)
 
 
 def _staged(a, b, mode, grouped=False):
-    """Whether the projection runs as the plain GEMM and the staged postprocess: where the GEMM's best
-    tile is smaller than a head (few rows: 128 x 7168 x 5376 INT8 14 us + 4 us against 26 us fused on
-    one-head tiles), or where gemm() may split K over 256-row tiles.  The fused kernel's tiles otherwise:
-    it takes the plain GEMM's choice between one-head and 256-row tiles.  Both give the plain GEMM's bits
-    through the postprocess.  The grouped layout (Q/K/V) is wide, so 256-row tiles hold their round and
-    K ranges with a second and a third pass over the output cost more than they save: 768 x 10752 x 1024
-    INT8 16.3 us fused against 27.3 us, 256 x 21504 x 1024 15.8 us against 22.0 us."""
-    tile = tile_plan(mode, a, b)
-    if tile == "256":
-        return not grouped and mode == "int8" and splitk_plan(a.shape[0], b.shape[0], a.shape[1]) > 1
-    return tile != "128"
+    m, k = a.shape
+    return hip.projection_staged(tile_plan(mode, a, b), mode, m, b.shape[0], k, grouped)
 
 
 def _epsilon(epsilon):
@@ -84,7 +76,7 @@ def projection_qk_rope(
     cos,
     sin,
     mode="int8",
-    tile=(32, 128, 4, 1),
+    tile=_TILE,
     *,
     a_scales=None,
     b_scales=None,
@@ -93,6 +85,11 @@ def projection_qk_rope(
     """Return BF16 [heads, M, 128] Q or K after projection, RMSNorm and RoPE
     (qk_rope.py:120-182).  A[M,K], B[N,K] INT8 with FP32 scales a_scales[M], b_scales[N],
     or BF16 when mode="bf16"; gamma BF16[128]; cos/sin BF16[M,R] rotate (d, d+R) for d < R."""
+    fast = hip._fast
+    if fast is not None and tile is _TILE and getattr(hip._override, "splits", None) is None:
+        y = fast.qk(a, b, gamma, cos, sin, mode, a_scales, b_scales, epsilon)
+        if y is not None:
+            return y
     if mode not in ("int8", "bf16"):
         raise NotImplementedError("Q/K projection fusion supports INT8 or BF16 only")
     if a.dim() != 2 or b.dim() != 2 or not all(a.shape) or not all(b.shape):
@@ -167,6 +164,11 @@ def projection_qkv_rope(a, w, q_gamma, k_gamma, cos, sin, mode="int8", *, a_scal
 
     Returns BF16 (Q, K, V), each [heads, M, 128].  Q and K get the per-head RMSNorm (q_gamma /
     k_gamma) and split-half RoPE of projection_qk_rope; V is the BF16-rounded projection."""
+    fast = hip._fast
+    if fast is not None and getattr(hip._override, "splits", None) is None:
+        qkv = fast.qkv(a, w, q_gamma, k_gamma, cos, sin, mode, a_scales, w_scales, epsilon)
+        if qkv is not None:
+            return qkv
     if mode not in ("int8", "bf16"):
         raise NotImplementedError("grouped Q/K/V projection supports INT8 or BF16 only")
     if a.dim() != 2 or w.dim() != 2 or not all(a.shape) or not all(w.shape):
