@@ -11,8 +11,9 @@
 // RMS moves only the scales (fold = true) and the row peak and statistics can share one
 // barrier.  One workgroup of 4 wave64 per row; a lane holds NCH chunks of EPC consecutive elements in
 // VGPRs.  B = 1 takes the same kernel without the butterflies where its chunks of 8 apply (K % 8 == 0,
-// aligned operands, K <= 16384); any other K, and operands without that alignment, read the row through
-// the cache element by element, once per pass ([512, 5376] BF16: 14.3 us, against 5.2 us in registers).
+// aligned operands, K <= 16384) and the row has enough of them to occupy the lanes; any other row is
+// read through the cache element by element, once per pass ([512, 5376] BF16: 14.3 us, against 5.2 us
+// in registers; [9914, 256]: 9.3 us, against 12.5 us with 32 of the 256 lanes at work).
 #include "hadamard_core.h"
 
 namespace m5k {
@@ -87,7 +88,7 @@ __device__ constexpr float transform_factor() {
   else return hadamard::inv_sqrt_block<B>();
 }
 
-// Register-resident rows (B >= 32: K % B == 0; B = 1: K % 8 == 0).
+// Register-resident rows (B >= 32: K % B == 0; B = 1: K % 8 == 0, K of 512 or 640 and more).
 template <int XDT, int B, int NCH, bool FOLD>
 __global__ __launch_bounds__(kThreads) void rms_quant_block_kernel(RmsParams p) {
   __shared__ float red[2 * kWaves];  // unfolded: statistics, then peak
@@ -255,8 +256,10 @@ template <int XDT, bool FOLD>
 int by_block(int block, const RmsParams& p, int64_t rows, hipStream_t st) {
   switch (block) {
     case 1:
-      if (p.k % 8 == 0 && p.k <= 8 * kThreads * 8 && aligned16(p.x) && aligned16(p.gamma) &&
-          (reinterpret_cast<uintptr_t>(p.signs) & 7u) == 0 && (reinterpret_cast<uintptr_t>(p.q) & 7u) == 0)
+      // The lines where both take the same time at 1024 to 9914 rows (16-bit: 9914 x 512 12.2 us element
+      // by element, 13.2 us in registers; x 768 15.9, 14.8.  FP32: x 384 11.2, 11.0; x 640 15.2, 12.0).
+      if (p.k >= (XDT == M5K_F32 ? 512 : 640) && p.k % 8 == 0 && p.k <= 8 * kThreads * 8 && aligned16(p.x) &&
+          aligned16(p.gamma) && (reinterpret_cast<uintptr_t>(p.signs) & 7u) == 0 && (reinterpret_cast<uintptr_t>(p.q) & 7u) == 0)
         return launch_block<XDT, 1, FOLD>(p, rows, st);
       rms_quant_plain_kernel<XDT, FOLD><<<dim3(static_cast<unsigned>(rows)), dim3(kThreads), 0, st>>>(p);
       return launch_status("m5k_rms_quantize");

@@ -1,5 +1,5 @@
-"""Unrotated RMS quantization (block 1): rows held in registers (K % 8 == 0, K <= 16384) against
-the element-by-element kernel, which the same row with one zero appended takes."""
+"""Unrotated RMS quantization (block 1): rows held in registers (K % 8 == 0, K from 640, FP32 512, to
+16384) against the element-by-element kernel, which the same row with one zero appended takes."""
 
 import pytest
 import torch
@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize("k", [8, 16, 2040, 2048, 2056, 5376, 8200, 16376, 16384])
+@pytest.mark.parametrize("k", [8, 16, 504, 512, 632, 640, 2040, 2048, 2056, 5376, 8200, 16376, 16384])
 def test_register_rows_equal_the_general_kernel(dtype, k, device):
     g = torch.Generator(device="cpu").manual_seed(k)
     x = torch.randn((7, k), generator=g).to(dtype)
