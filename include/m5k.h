@@ -213,7 +213,8 @@ int m5k_gemm_schedule_state(void);
  *   4  16 columns per workgroup, K over eight waves (m <= 32).
  * INT8 results are bit-identical under every tile.  Float results (FP32 sums) are the same bits for
  * tiles 1 to 3, and for tile 0 under every schedule; between these groups and tile 4 the order of the
- * sum differs.  Float rows of under 1 KiB always take tile 0.
+ * sum differs.  Aligned float rows of under 1 KiB always take tile 0.  Unaligned I8 rows of at most
+ * 128 bytes run on 256 x 256 tiles where the tile reported here would take several rounds longer.
  * max_splits (1..64, more than 1 for I8 and U8 only) offers K ranges of tiles 1 to 3 too; *splits
  * receives how many the choice takes (1: no partial sums; tiles 0 and 4 always).  K ranges of
  * 256-row tiles are not weighed here: m5k_gemm_split_plan has the split entry points' whole choice.

@@ -247,6 +247,16 @@ inline plan::Choice plan_tile(int mode, int64_t m, int64_t n, int64_t kb, int cu
   return plan::choose(m, n, kb, cus, aligned, max_splits, limit_us);
 }
 
+// Unaligned INT8 rows of one stage (K <= 128): the byte-wise 256-row loop costs one pass there, 3 + 17.5 us
+// a round, and over several rounds of small tiles `small` less than they do (4096 x 4096 x 100: 21.4 us
+// against 29.2; 9000 x 1600 x 65 20.5 against 26.2).  From two stages on the small tiles are ahead (x 257:
+// 34.3 us against 46.4).
+inline bool one_stage_on_256(int mode, bool aligned, int64_t m, int64_t n, int64_t kb, int cus, const plan::Choice& small) {
+  if (mode != I8 || aligned || kb > BKB || cus <= 0) return false;
+  const int64_t rounds = plan::ceil_div(plan::ceil_div(m, BM) * plan::ceil_div(n, BN), cus);
+  return 3.0 + 17.5 * static_cast<double>(rounds) < 0.95 * small.us;
+}
+
 template <class C, bool ALIGNED, int OUT_DT, int BIAS, int GATE>
 int launch_ring(const uint8_t* A, const uint8_t* B, int64_t m, int64_t n, int64_t kb, const EpiParams& q,
                 hipStream_t st, const char* name) {
@@ -297,7 +307,7 @@ int launch(const void* a, const void* b, int64_t m, int64_t n, int64_t k, const 
   q.coalesced = n % 8 == 0 && aligned16(p.c) && (p.residual == nullptr || (aligned16(p.residual) && aligned16(p.gate)));
   if constexpr (small_mode(MODE) && !RAW) {
     const plan::Choice small = plan_tile(MODE, m, n, kb, device_cus(), aligned);
-    if (small.tile != plan::TILE_256)
+    if (small.tile != plan::TILE_256 && !one_stage_on_256(MODE, aligned, m, n, kb, device_cus(), small))
       return launch_small<MODE, OUT_DT, BIAS, GATE>(small.tile, aligned, A, B, m, n, kb, q, st, name);
   }
   if (aligned) {
@@ -329,7 +339,8 @@ int launch(const void* a, const void* b, int64_t m, int64_t n, int64_t k, const 
     } else {
       launch_kernel(gemm_kernel<MODE, true, OUT_DT, BIAS, GATE, RAW>, grid, block, st, A, B, (int)m, (int)n, kb, q);
     }
-  } else if constexpr (RAW || MODE == F8 || MODE == F32) {
+  } else if constexpr (MODE == I8 || MODE == F8 || MODE == F32) {
+    // INT8: one stage, no CU count, or the raw accumulators.
     launch_kernel(gemm_kernel<MODE, false, OUT_DT, BIAS, GATE, RAW>, grid, block, st, A, B, (int)m, (int)n, kb, q);
   } else {
     return launch_small<MODE, OUT_DT, BIAS, GATE>(plan::TILE_64, false, A, B, m, n, kb, q, st, name);

@@ -108,6 +108,26 @@ def test_unaligned_rows_bit_exact(m, n, k, device):
     assert torch.all((gemm(x, w, "bf16").double() - exact).abs() <= (k + 4) * 2.0**-24 * 1.01 * size)
 
 
+@pytest.mark.parametrize("k", [65, 100, 127])
+@pytest.mark.parametrize("m,n", [(2305, 6017), (4096, 4096)])
+def test_unaligned_rows_of_one_stage_over_many_tiles(m, n, k, device):
+    """256-row tiles there, a partial tile on both sides.  |sum a b| <= 127 * 127 * 127 < 2^24, so the FP32
+    product of the codes is exact, and the epilogue is its FP32 sequence."""
+    print(f"case m={m} n={n} k={k}", flush=True)
+    g = torch.Generator(device="cpu").manual_seed(m + n + k)
+    a, b, sa, sb = _int8(g, m, n, k, device)
+    acc = a.float() @ b.float().T
+    bias = torch.randn((n,), generator=g).to(device)
+    res = torch.randn((m, n), generator=g).bfloat16().to(device)
+    scaled = (acc * sa[:, None]) * sb
+    kw = dict(a_scales=sa, b_scales=sb)
+    assert torch.equal(gemm(a, b, "int8", **kw), scaled)
+    assert torch.equal(gemm(a, b, "int8", output_dtype=torch.bfloat16, **kw), scaled.bfloat16())
+    assert torch.equal(gemm(a, b, "int8", bias=bias, **kw), scaled + bias)
+    gated = gemm(a, b, "int8", residual=res, gate=bias.bfloat16(), output_dtype=torch.bfloat16, **kw)
+    assert torch.equal(gated, (res.float() + scaled.bfloat16().float() * bias.bfloat16().float()).bfloat16())
+
+
 @pytest.mark.parametrize("offset", [1, 2, 7, 8, 15])
 def test_unaligned_bases_bit_exact(offset, device):
     """16-byte rows whose first byte is not 16-byte aligned (a view into a larger buffer); the last
