@@ -779,7 +779,7 @@ struct TileScalePrefetch {
 // scales from the LDS one block row at a time, so the epilogue holds few extra registers.
 template <class G>
 struct TileScales {
-  const float* s;  // rows [0, BM), then columns [BM, G::TM + G::TN)
+  const float* s;  // rows [0, G::TM), then columns [G::TM, G::TM + G::TN)
   __device__ __forceinline__ TileScales(const float* __restrict__ sa, const float* __restrict__ sb, int M, int N,
                                         int m0, int n0, int tid, uint8_t* lds = g_lds) {
     float* w = reinterpret_cast<float*>(lds + EpiLayout<G>::SCALES_OFFSET);

@@ -8,7 +8,9 @@
 //   gated      branch = bf16(value); C = bf16(float(Residual) + float(branch) * float(Gate[..]))
 //   float      C = O(float(acc))
 // The library is compiled with -ffp-contract=off so none of these products and sums is
-// fused into an FMA: the FP32 rounding sequence is exactly the one written above.
+// fused into an FMA: the FP32 rounding sequence is exactly the one written above.  For FP16 outputs the
+// compiler joins the last FP32 operation and the cast into one v_fma_mixlo_f16, which rounds once: such
+// an output can lie one FP16 step from the rounded FP32 one (the same in every kernel of this library).
 #pragma once
 #include "gemm_core.h"
 

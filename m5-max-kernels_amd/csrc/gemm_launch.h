@@ -230,8 +230,9 @@ inline double units_256(bool md16, int64_t m, int64_t n, int cus) {
 
 // The tile of an [m, n] output with rows of kb bytes (no partial sums): one of gemm_plan.h's, or
 // TILE_256 for the 256-row schedules.  Aligned operands under a forced schedule run that schedule.
-// Float rows of under 1 KiB stay there too: the smaller tiles split K over waves, and eight 128-byte
-// lines leave each of them one or none.  FP8's unaligned operands keep the register-staged loop.
+// Aligned float rows of under 1 KiB stay there too: the smaller tiles split K over waves, and eight
+// 128-byte lines leave each of them one or none.  Unaligned operands have ring tiles at any K, except
+// FP8's, which keep the register-staged loop (one_stage_on_256: INT8's of one stage, over many tiles).
 inline plan::Choice plan_tile(int mode, int64_t m, int64_t n, int64_t kb, int cus, bool aligned, int max_splits = 1,
                               double limit_us = 1e30) {
   const plan::Choice none{plan::TILE_256, 1, 0.0};

@@ -1,8 +1,12 @@
 // Host-side choice of a GEMM's tile (no device code).
 //
-// Times are microseconds on MI355X as functions of the row length in bytes, fitted to sweeps of
-// INT8, FP8 and BF16 products (M 1 to 2048, N 256 to 28672, rows of 256 bytes to 28 KiB); they
-// predict the sweeps within about 15%.  A round is one pass of workgroups over the CUs.
+// Times are microseconds on MI355X as functions of the row length in bytes, fitted to INT8, FP8 and BF16
+// products with a weight that the Infinity Cache holds.  Over M 1 to 2048, N 1024 to 21504 and K 1024 to
+// 16384 (about 750 products a mode) four in five lie within 15% of them; with weights read from memory
+// just over half do: the 64-row tiles take a fifth longer, the decode tile and K ranges about as
+// modelled.  The choice costs 1% (weights from memory: 2%) over the fastest launch in the geometric
+// mean, at worst 1.3 and 1.4 times.
+// A round is one pass of workgroups over the CUs.
 //
 //   128 x 128 ring     1 workgroup per CU:   2 + r (6 + 3.6 us/KB)   1024 x 4096 x 4096 INT8 21.5 us
 //                      from 3 rounds on, 15% more (8366 x 1920 x 8192 INT8, 4 rounds: 200 us)

@@ -10,8 +10,8 @@
 // their accumulators through the LDS, and each wave finishes a quarter-height strip: the geometry
 // of Grid<4, 2, TN, TM>, whose epilogue runs unchanged.
 //
-// NST stages ring through the LDS, all but the one being read in flight: 24 to 48 KiB of weights per CU
-// under way against 16 KiB for the 256-row tiles' two-stage loop, which is what a short-M product,
+// NST stages (2 to 4) ring through the LDS, all but the one being read in flight: 32 to 48 KiB of weights
+// per CU under way against 16 KiB for the 256-row tiles' two-stage loop, which is what a short-M product,
 // bound by streaming the weight, needs.  INT8, us, 256-row tiles (split over K with a second pass for
 // the partial sums where that paid) against these, unsplit: 128 x 4096 x 4096 16.2 -> 9.7; 128 x 5376
 // x 14336 31.1 -> 24.3; 512 x 7168 x 5376 36.1 -> 25.2; 128 x 21504 x 5376 49.7 -> 33.5; 1024 x 4096

@@ -13,8 +13,8 @@
 // contraction).
 //
 // The fused kernels run the GEMM main loop for a 256-row x 2-head tile (qk_ring_kernel: a 128-row x
-// one-head tile), stage the BF16 projection in the (then free) LDS, and normalize each (row, head) with a group
-// of 16 lanes (8 channels each, one 16-byte read and one 16-byte head-major store per lane).
+// one-head tile), stage the BF16 projection in the (then free) LDS, and normalize each (row, head) with
+// a group of 16 lanes (8 channels each, one 16-byte read and one 16-byte head-major store per lane).
 // The staged kernel runs the same per-(row, head) routine on a BF16 [M,N] projection in HBM,
 // so the two paths agree bit for bit whenever their projections do.
 #include "gemm_launch.h"
@@ -291,7 +291,8 @@ __device__ __forceinline__ void qk_tile_epilogue(const AccTile<MODE, G>& acc, in
   // words spilled 35 VGPRs to scratch; this form uses 228 VGPRs and no scratch, same bits (C5
   // fused projection 162.6 -> 160.2 us, one box).
   LaneRope lr, lrk;  // Q (or single-projection) gamma; K gamma in the grouped layout
-  constexpr int LOOKAHEAD = ROWS_PER_GROUP < 4 ? ROWS_PER_GROUP : 4;  // rows of cos/sin in flight ahead of the row being rotated
+  // Rows of cos/sin in flight ahead of the row being rotated.
+  constexpr int LOOKAHEAD = ROWS_PER_GROUP < 4 ? ROWS_PER_GROUP : 4;
   uint4 cw[ROWS_PER_GROUP], sw[ROWS_PER_GROUP];
   int row0 = m0 + group;
   __asm__ volatile("" : "+v"(row0));
@@ -517,7 +518,8 @@ int launch_fused(const void* a, const void* b, int64_t m, int64_t n, int64_t k, 
   auto* B = static_cast<const uint8_t*>(b);
   const int fast = fast_rope(p);
   // The plain GEMM's choice for this product.  Where it runs on ring tiles, so does this kernel, whose
-  // float sums then have the plain GEMM's bits.
+  // float sums then have the plain GEMM's bits.  There is no fused decode tile: where the plain GEMM
+  // takes it, BF16 sums here are the 256-row tiles' (the Python wrapper runs those sizes staged).
   const int tile = gemm::detail::plan_tile(MODE, m, n, kb, device_cus(), aligned).tile;
   if (!aligned || tile == gemm::plan::TILE_128 || tile == gemm::plan::TILE_64 || tile == gemm::plan::TILE_64_DEEP) {
     using R = gemm::detail::RingTiles<MODE>;

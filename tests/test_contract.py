@@ -282,9 +282,9 @@ def test_tail_split_plan_decisions():
     assert splitk_plan(1024, 5376, 14336) == 3 and splitk_plan(1024, 4096, 16384) == 4
     assert splitk_plan(1536, 5376, 14336) == 1 and splitk_plan(2048, 4096, 16384) == 1
     assert splitk_plan(1024, 5376, 14336, skinny=False) == 3
-    # Two tile rows: 256 x 64 split tiles while 2 * ceil(N / 64) * splits fits one round.
+    # Two tile rows: ranges counted in 256 x 64 columns while 2 * ceil(N / 64) * splits fits one round.
     assert splitk_plan(512, 4096, 4096) == 2 and splitk_plan(512, 1536, 5376) == 5
-    # One tile row, K <= 8192: split counts sized to 256 x 64 tiles (64 columns at N 4096).
+    # One tile row, K <= 8192: counted in 256 x 64 columns (64 of them at N 4096).
     assert splitk_plan(128, 4096, 4096) == 4 and splitk_plan(1, 4096, 4096) == 4
     assert splitk_plan(128, 7168, 5376) == 2 and splitk_plan(128, 1536, 5376) == 10
     # 224 columns of 64 need two rounds even at 2 splits: 256 x 128 tiles (112 columns) take

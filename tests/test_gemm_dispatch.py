@@ -72,7 +72,7 @@ def test_each_tuner_launch_reaches_its_entry_point(recorder, m, n, k):
 
 
 def test_short_m_plan_splits_but_forced_plain_does_not(recorder):
-    # attn_q.m128: the library's plan splits K; the forced "plain" launch must not.
+    # attn_q.m128: gemm() goes to the split entry point; under the forced "plain" schedule it must not.
     assert hip.splitk_plan(128, 7168, 5376, 256) > 1
     a = torch.zeros((128, 5376), dtype=torch.int8)
     b = torch.zeros((7168, 5376), dtype=torch.int8)
@@ -102,8 +102,9 @@ def test_set_schedule_rejects_unknown_codes():
 
 
 def test_fp8_short_m_splits_k_and_large_m_or_forced_plain_does_not(recorder):
-    # h3 ffn_down at M = 128: 21 tiles of 256 x 256 leave most CUs idle, so the FP8 GEMM splits K
-    # over 256 x 128 tiles; at M = 4096, and under a forced schedule, it runs unsplit.
+    # h3 ffn_down at M = 128: 21 tiles of 256 x 256 leave most CUs idle, so the FP8 GEMM goes to the
+    # split entry point, with room for K ranges of 256 x 128 tiles; at M = 4096, and under a forced
+    # schedule, it goes to the plain one.
     m, n, k = 128, 5376, 14336
     planned = hip.splitk_plan(m, n, k, 256, skinny=False)
     assert planned > 1 and -(-n // 128) * planned <= 256

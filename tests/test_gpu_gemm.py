@@ -1,6 +1,6 @@
 """GPU parity of the MFMA GEMMs (m5k_gemm_i8 / _i8_acc / _f8 / _float).
 
-Bars (north-star targets): INT32 accumulators bit-exact; W8A8 BF16/FP32 outputs
+Bars: INT32 accumulators bit-exact; W8A8 BF16/FP32 outputs
 bit-exact against the oracle's FP32 epilogue (hence well within 1 bf16 ulp); FP8 and
 float modes within the reference's rel-L2 gate 0.008 of float64 (tests/test_metal.py:85-112
 of the reference) and rel-L2 1e-3 of the float64 product for FP32 output.

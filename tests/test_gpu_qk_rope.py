@@ -3,8 +3,8 @@ staged postprocess (m5k_qk_norm_rope).
 
 Bars: INT8 fused == staged (quantize -> gemm bf16 -> qk_norm_rope) bit for bit, as the reference
 requires (tests/test_qk_rope_metal.py:78-81 of the reference), and here also for BF16 since both
-paths share one main loop; both within rel-L2 1e-3 of the float64 reference fed the exact
-projection (the north-star RoPE bar; the reference's own gate is 0.008).
+take the plain GEMM's order of sums; both within rel-L2 1e-3 of the float64 reference fed the exact
+projection (the reference's own gate is 0.008).
 """
 
 from __future__ import annotations
