@@ -306,7 +306,8 @@ PyObject* project(PyObject* const* args, bool grouped) {
   } else if (args[at + 3] != Py_None || args[at + 4] != Py_None) {
     Py_RETURN_NONE;
   }
-  const at::Tensor *g = plain(args[2]), *gk = grouped ? plain(args[3]) : g, *cos = plain(args[at]), *sin = plain(args[at + 1]);
+  const at::Tensor *g = plain(args[2]), *gk = grouped ? plain(args[3]) : g;
+  const at::Tensor *cos = plain(args[at]), *sin = plain(args[at + 1]);
   if (!vector_of(g, HEAD, at::kBFloat16, dev) || !vector_of(gk, HEAD, at::kBFloat16, dev) || !aligned16(g->data_ptr()) ||
       !aligned16(gk->data_ptr()))
     Py_RETURN_NONE;

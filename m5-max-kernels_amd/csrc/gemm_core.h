@@ -672,8 +672,8 @@ __device__ __forceinline__ void mainloop_dma(const uint8_t* __restrict__ A, cons
 
 // Register-staged main loop for operands that the direct-to-LDS loads do not take, in the forms
 // that the ring kernels (gemm_ring.h) do not serve, or serve slower: FP32, FP8 at a misaligned base, the
-// raw INT32 accumulators, and INT8 rows of one stage over many tiles.  Bytes are loaded one at a time with exact bounds, then stored to the same swizzled
-// layout.
+// raw INT32 accumulators, and INT8 rows of one stage over many tiles.  Bytes are loaded one at a time
+// with exact bounds, then stored to the same swizzled layout.
 template <int MODE, class G>
 __device__ __forceinline__ void mainloop_staged(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, int M,
                                                 int N, int64_t Kb, int tile_m0, int tile_n0, AccTile<MODE, G>& acc) {

@@ -259,7 +259,8 @@ int by_block(int block, const RmsParams& p, int64_t rows, hipStream_t st) {
       // The lines where both take the same time at 1024 to 9914 rows (16-bit: 9914 x 512 12.2 us element
       // by element, 13.2 us in registers; x 768 15.9, 14.8.  FP32: x 384 11.2, 11.0; x 640 15.2, 12.0).
       if (p.k >= (XDT == M5K_F32 ? 512 : 640) && p.k % 8 == 0 && p.k <= 8 * kThreads * 8 && aligned16(p.x) &&
-          aligned16(p.gamma) && (reinterpret_cast<uintptr_t>(p.signs) & 7u) == 0 && (reinterpret_cast<uintptr_t>(p.q) & 7u) == 0)
+          aligned16(p.gamma) && (reinterpret_cast<uintptr_t>(p.signs) & 7u) == 0 &&
+          (reinterpret_cast<uintptr_t>(p.q) & 7u) == 0)
         return launch_block<XDT, 1, FOLD>(p, rows, st);
       rms_quant_plain_kernel<XDT, FOLD><<<dim3(static_cast<unsigned>(rows)), dim3(kThreads), 0, st>>>(p);
       return launch_status("m5k_rms_quantize");

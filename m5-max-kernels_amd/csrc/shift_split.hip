@@ -13,9 +13,9 @@
 // 5.2 TB/s for [7168, 5376]), so 16-bit operands are read as they are and converted in registers; FP32
 // copies of them took 38 us to make and 25 us to read, against 15 us.  One wave owns one W row; each
 // lane streams 8-element chunks (16-byte loads), multiplies them into up to kPB conditioning rows held
-// in registers, and the wave sums its lanes with the fixed DPP tree.  Up to kPB rows this reads W once.  More conditioning rows
-// make the projection a small GEMM, [P, K] x [N, K]^T, which runs on the BF16/F16/FP32 MFMA
-// GEMM with FP32 output instead (W read once per 256-row tile of P).
+// in registers, and the wave sums its lanes with the fixed DPP tree.  Up to kPB rows this reads W once.
+// More conditioning rows make the projection a small GEMM, [P, K] x [N, K]^T, which runs on the
+// BF16/F16/FP32 MFMA GEMM with FP32 output instead (W read once per 256-row tile of P).
 #include "m5k_common.h"
 
 namespace m5k {

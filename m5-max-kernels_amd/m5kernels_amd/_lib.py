@@ -107,10 +107,10 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
 
 
 def load_fast():
-    """The native front of quantize(), gemm() and the projections (binding/fast_ops.cpp), linked against libm5k.so, or
-    None where the libraries have not been built.  One that does not load, or that was compiled for
-    another C ABI or another torch (left from an older build), warns: the same kernels then run with
-    the checks in Python."""
+    """The native front of quantize(), gemm() and the projections (binding/fast_ops.cpp), linked
+    against libm5k.so, or None where the libraries have not been built.  One that does not load, or
+    that was compiled for another C ABI or another torch (left from an older build), warns: the same
+    kernels then run with the checks in Python."""
     if not (FAST_PATH.exists() and LIB_PATH.exists()) or _current_raw_stream is None:
         return None
     spec = importlib.util.spec_from_file_location("m5k_fast", FAST_PATH)
